@@ -265,7 +265,7 @@ def bench_variants(torch, S, L, stream, reps=10):
         "fp16_floor_us": round(NS3 * H3 * NP3 * 2 * hd3 * 2 / (HBM_PEAK_GBS * 1e3), 1),
         "layout": f"{NS3} sequences x {NP3} positions x {H3} heads (MHA), hd {hd3}, K 5/4/4 + V 5 records "
                   f"({kB3} + {vB3} B); per layer step: one batched fused attention call "
-                  f"(sp_hip_attn_decode_seqs, one-position-per-lane kernel); step_layer_us_16_calls: "
+                  f"(sp_hip_attn_decode_seqs, matrix-core kernel); step_layer_us_16_calls: "
                   f"{NS3} single-sequence calls"}
     c3d.free()
     del x, y

@@ -216,9 +216,9 @@ size_t sp_hip_attn_noalloc_max_floats(void);
  * own queries d_q[s] ([n_seq][n_q][head_dim] fp32): d_out [n_seq][n_q][head_dim] and
  * d_scores, sequence s's [n_q][seq_len[s]] block starting at element
  * n_q * (seq_len[0] + ... + seq_len[s-1]). Results equal n_seq separate calls over those
- * ranges. The hd 96 (K 5/4/4, V 5) and hd 64 (K 5/5/4/3, V 3) layouts run every sequence
- * in one launch each of the query preparation, the split kernel and the combine (workspace
- * grown on demand); other layouts run the single-sequence kernels once per sequence. */
+ * ranges. The matrix-core layouts (K 5/4/4 with V 5 at head_dim 64 and 96, K 5/5/4/3 with V 3
+ * at head_dim 64, 128 and 256) run every sequence in one launch, in the workspace sized at
+ * init; other layouts run the general kernels once per sequence. */
 int sp_hip_attn_decode_seqs(const sp_hip_cache_t *cc, int layer, int n_seq, const int *seq_start,
                             const int *seq_len, const float *d_q, int n_q, float kq_scale, float *d_scores,
                             float *d_out, void *stream);

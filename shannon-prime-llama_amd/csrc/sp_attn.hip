@@ -18,6 +18,7 @@
 //   3. k_attn_combine: merge splits (log-sum-exp), one inverse VHT2 per head.
 // No full-precision K or V is materialized anywhere.
 #include <stdlib.h>
+#include <string.h>
 
 #include "sp_internal.h"
 
@@ -243,94 +244,19 @@ k_attn_combine(const SpPlan VP, const float *__restrict__ ws, int n_splits, int 
         for (int k = tid; k < hd; k += SP_WAVE) out[(long long)h * hd + k] = c[k];
 }
 
-// The same merge for rows of at most 64 splits by one wave per row: split `lane`'s m and
-// l, a wave-wide max and sum (lane shuffles), the row's elements by lane (i = lane,
-// lane + 64, ...), each summed over the splits in order, then the inverse transform.
-// A batch of short sequences has a few splits per row, so the 1024-thread block of
-// k_attn_combine would be mostly idle and its block reductions the cost.
-__global__ void __launch_bounds__(64)
-k_attn_combine_wave(const SpPlan VP, const float *__restrict__ ws, int n_splits, int hd, float *__restrict__ out) {
-    __shared__ float e_s[SP_WAVE];
-    __shared__ float c[ATT_MAX_HD];
-    const int h = blockIdx.x, lane = threadIdx.x;
-    const long long row = hd + 2;
-    const float *base = ws + (long long)h * n_splits * row;
-    const bool live = lane < n_splits;
-    const float m = live ? base[lane * row] : -INFINITY;
-    const float lv = live ? base[lane * row + 1] : 0.0f;
-    // rows of at most CW splits (a batch of short sequences) load their elements at
-    // entry with m and l, so the row waits on memory once; longer rows load them in the
-    // sum below (their loads at entry measured slower)
-    constexpr int CW = 8, EPL = ATT_MAX_HD / SP_WAVE;
-    const bool pre = n_splits <= CW;
-    float pv[CW][EPL];
-    if (pre) {
-#pragma unroll
-        for (int sp = 0; sp < CW; sp++) {
-#pragma unroll
-            for (int u = 0; u < EPL; u++) {
-                const int i = lane + u * SP_WAVE;
-                pv[sp][u] = sp < n_splits && i < hd ? base[sp * row + 2 + i] : 0.0f;
-            }
-        }
-    }
-    float M = m;
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) M = fmaxf(M, __shfl_xor(M, o, SP_WAVE));
-    const float e = live ? __expf(m - M) : 0.0f;
-    float L = lv * e;
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) L += __shfl_xor(L, o, SP_WAVE);
-    e_s[lane] = e;
-    __syncthreads();
-    const float invL = 1.0f / L;
-    if (pre) {
-#pragma unroll
-        for (int u = 0; u < EPL; u++) {
-            const int i = lane + u * SP_WAVE;
-            if (i >= hd) continue;
-            float acc = 0.0f;
-#pragma unroll
-            for (int sp = 0; sp < CW; sp++)
-                if (sp < n_splits) acc = fmaf(pv[sp][u], e_s[sp], acc);
-            c[i] = acc * invL;
-        }
-    } else {
-        for (int i = lane; i < hd; i += SP_WAVE) {
-            float acc = 0.0f;
-#pragma unroll 8
-            for (int sp = 0; sp < n_splits; sp++) acc = fmaf(base[sp * row + 2 + i], e_s[sp], acc);
-            c[i] = acc * invL;
-        }
-    }
-    __syncthreads();
-    sp_transform_lds(c, hd, VP, lane);
-    for (int k = lane; k < hd; k += SP_WAVE) out[(long long)h * hd + k] = c[k];
-}
-
-hipError_t sp_launch_attn_lane_seqs(const SpPlan &KP, const SpPlan &VP, const int *order, const SpAttnArgs &A,
-                                    const SpSeqTab &T, float *ws, size_t ws_floats, int n_runs, hipStream_t s) {
-    const size_t n_rows = (size_t)T.n_seq * A.n_q;
-    if (T.n_seq < 1 || T.n_seq > SP_ATTN_MAX_SEQ || n_runs <= 0 || n_runs > ATT_MAX_SPLITS ||
-        n_rows * A.hd + n_rows * n_runs * (A.hd + 2) > ws_floats)
-        return hipErrorInvalidValue;
-    float *qt = ws;
-    float *part = ws + n_rows * A.hd;
-    hipLaunchKernelGGL(k_attn_prep, dim3((unsigned)n_rows), dim3(64), 0, s, KP, order, A.q, A.hd, A.kq_scale, qt);
-    const hipError_t le = sp_launch_attn_lane_split(KP, VP, A, T, qt, part, n_runs, s);
-    if (le != hipSuccess) return le;
-    if (A.out && n_runs <= SP_WAVE)
-        hipLaunchKernelGGL(k_attn_combine_wave, dim3((unsigned)n_rows), dim3(SP_WAVE), 0, s, VP, part, n_runs, A.hd,
-                           A.out);
-    else if (A.out)
-        hipLaunchKernelGGL(k_attn_combine, dim3((unsigned)n_rows), dim3(COMB_THREADS), 0, s, VP, part, n_runs, A.hd,
-                           A.out);
-    return hipGetLastError();
-}
-
 size_t sp_attn_workspace_floats(int n_q, int hd, int max_kv) {
     const int n_splits = (max_kv + ATT_CHUNK - 1) / ATT_CHUNK;
     return (size_t)n_q * hd + (size_t)n_q * n_splits * (hd + 2) + SP_ATTN_COUNTERS + SP_ATTN_COUNTER_STRIDE;
+}
+
+hipError_t sp_launch_attn_wave_ws(const SpPlan &KP, const SpPlan &VP, const int *order, const SpAttnArgs &A,
+                                  const SpSeqTab &T, float *workspace, size_t ws_floats, hipStream_t s) {
+    if (ws_floats < SP_ATTN_COUNTERS + SP_ATTN_COUNTER_STRIDE) return hipErrorInvalidValue;
+    // the arrival counters: the workspace's last SP_ATTN_COUNTERS words (plus up to one
+    // line of slack), starting on a 256-byte boundary
+    const size_t part_floats = ws_floats - SP_ATTN_COUNTERS - SP_ATTN_COUNTER_STRIDE;
+    int *cnt = reinterpret_cast<int *>(((uintptr_t)(workspace + part_floats) + 255) & ~(uintptr_t)255);
+    return sp_launch_attn_wave(KP, VP, order, A, T, workspace, part_floats, cnt, s);
 }
 
 hipError_t sp_launch_attn_decode(const SpPlan &KP, const SpPlan &VP, const int *order,
@@ -344,32 +270,13 @@ hipError_t sp_launch_attn_decode(const SpPlan &KP, const SpPlan &VP, const int *
     float *qt = workspace;
     float *part = workspace + (size_t)A.n_q * A.hd;
     const int want_out = A.out != nullptr;
-    {
-        // the per-KV-head arrival counters: the workspace's last SP_ATTN_COUNTERS words
-        // (plus up to one line of slack), starting on a 256-byte boundary
-        const uintptr_t ctail = (uintptr_t)(workspace + ws_floats - SP_ATTN_COUNTERS - SP_ATTN_COUNTER_STRIDE);
-        int *cnt = reinterpret_cast<int *>((ctail + 255) & ~(uintptr_t)255);
-        const hipError_t we = sp_launch_attn_wave(
-            KP, VP, order, A, part, ws_floats - (size_t)A.n_q * A.hd - SP_ATTN_COUNTERS - SP_ATTN_COUNTER_STRIDE, cnt, s);
-        if (we != hipErrorNotSupported) return we;
-    }
-    {
-        // hd 96 / hd 64 shipping layouts: the one-position-per-lane split kernel
-        // (sp_attn_lane.hip) between the same query preparation and combine
-        // (SP_HIP_NO_LANE_ATTN=1, read at each call, keeps them on the kernel below)
-        const char *off = getenv("SP_HIP_NO_LANE_ATTN");
-        const size_t part_floats = ws_floats - (size_t)A.n_q * A.hd - SP_ATTN_COUNTERS - SP_ATTN_COUNTER_STRIDE;
-        const int n_runs = (off && off[0] == '1') ? 0 : sp_attn_lane_runs(KP, VP, A, part_floats);
-        if (n_runs > 0) {
-            SpSeqTab T;
-            T.n_seq = 1;
-            T.max_len = A.n_kv;
-            T.start[0] = 0;
-            T.len[0] = A.n_kv;
-            T.soff[0] = 0;
-            return sp_launch_attn_lane_seqs(KP, VP, order, A, T, workspace, ws_floats, n_runs, s);
-        }
-    }
+    SpSeqTab T;
+    memset(&T, 0, sizeof(T));
+    T.n_seq = 1;
+    T.max_len = A.n_kv;
+    T.len[0] = A.n_kv;
+    const hipError_t we = sp_launch_attn_wave_ws(KP, VP, order, A, T, workspace, ws_floats, s);
+    if (we != hipErrorNotSupported) return we;
     hipLaunchKernelGGL(k_attn_prep, dim3(A.n_q), dim3(64), 0, s, KP, order, A.q, A.hd, A.kq_scale, qt);
     const size_t lds = (size_t)((ATT_CHUNK * A.kB + 8 + 15) & ~15) + (size_t)ATT_CHUNK * A.vB + 8;
     hipLaunchKernelGGL(k_attn_split, dim3(A.n_kvh, n_splits), dim3(256), lds, s, KP, VP, A, qt, part,

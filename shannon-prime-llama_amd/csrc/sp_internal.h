@@ -348,6 +348,7 @@ struct SpAttnArgs {
     long long k_head_stride, v_head_stride;  // bytes between KV heads
     int kB, vB;
     int n_kv, n_q, n_kvh, hd;
+    int start;          // first position (the matrix-core kernel's single-sequence launches)
     float kq_scale;
     const float *q;     // [n_q][hd]
     float *scores;      // [n_q][n_kv] or null
@@ -357,17 +358,6 @@ hipError_t sp_launch_attn_decode(const SpPlan &KP, const SpPlan &VP, const int *
                                  const SpAttnArgs &A, float *workspace, size_t ws_floats,
                                  hipStream_t s);
 size_t sp_attn_workspace_floats(int n_q, int hd, int max_kv);
-// One-position-per-lane split kernel for the hd 96 (K 5/4/4, V 5) and hd 64 (K 5/5/4/3,
-// V 3) layouts (sp_attn_lane.hip): runs per KV head that fit part_floats (0: no lane
-// kernel for these layouts), and the launch writing [m, l, o~[hd]] per (query head, run).
-int sp_attn_lane_runs(const SpPlan &KP, const SpPlan &VP, const SpAttnArgs &A, size_t part_floats, int n_seq = 1);
-hipError_t sp_launch_attn_lane_split(const SpPlan &KP, const SpPlan &VP, const SpAttnArgs &A, const SpSeqTab &T,
-                                     const float *qt, float *part, int n_runs, hipStream_t s);
-// Batched decode attention through the query preparation, the lane split kernel and the
-// combine (hd 96 / hd 64 layouts): q, out [n_seq][n_q][hd], scores at T.soff;
-// ws holds n_seq * n_q * hd prepared-query floats, then the partials.
-hipError_t sp_launch_attn_lane_seqs(const SpPlan &KP, const SpPlan &VP, const int *order, const SpAttnArgs &A,
-                                    const SpSeqTab &T, float *ws, size_t ws_floats, int n_runs, hipStream_t s);
 // Checks the arguments of a decode-attention call on one layer of a ship cache
 // and fills its launch arguments and K/V plans (band limit applied); -1 with the
 // error message set for bad arguments (sp_runtime.cpp).
@@ -377,18 +367,22 @@ int sp_attn_prepare(const sp_hip_cache_t *cc, int layer, int n_kv, const float *
 // Sets the message sp_hip_last_error() returns (sp_runtime.cpp).
 void sp_set_error(const char *fmt, ...);
 // Words at the end of every attention workspace (sp_attn_workspace_floats) that
-// hold the wave kernel's per-KV-head arrival counters, one per 256-byte line
-// (SP_ATTN_COUNTER_STRIDE words) so the KV heads' atomics do not queue on one
-// line: zero when the workspace is created, and back at zero after each call.
+// hold the matrix-core kernel's arrival counters, one per KV head and sequence of a launch on
+// a 256-byte line of its own (SP_ATTN_COUNTER_STRIDE words), so that their atomics do not
+// queue on one line: zero when the workspace is created, and back at zero after each call.
 #define SP_ATTN_COUNTER_STRIDE 64
 #define SP_ATTN_MAX_KVH 256
 #define SP_ATTN_COUNTERS (SP_ATTN_MAX_KVH * SP_ATTN_COUNTER_STRIDE)
-// Wave-tiled matrix-core kernel for the same layout (sp_attn_wave.hip): scores
-// and/or the attention output in one launch (each block writes a spectral-domain
-// partial [m, l, o~[hd]] per query head, at most part_floats floats, and the last
-// block of each KV head merges them); hipErrorNotSupported for other layouts.
-hipError_t sp_launch_attn_wave(const SpPlan &KP, const SpPlan &VP, const int *order, const SpAttnArgs &A, float *part,
-                               size_t part_floats, int *counters, hipStream_t s);
+// Matrix-core kernel (sp_attn_wave.h) over T's sequences: scores and/or the attention
+// output, in one launch for as many sequences as the counters and `part` hold (each block
+// writes a spectral-domain partial [m, l, o~[hd]] per query head and the last block of
+// each sequence's KV head merges them); hipErrorNotSupported for other layouts. A.q and
+// A.out hold T.n_seq blocks of n_q rows, A.n_kv is not read.
+hipError_t sp_launch_attn_wave(const SpPlan &KP, const SpPlan &VP, const int *order, const SpAttnArgs &A, const SpSeqTab &T,
+                               float *part, size_t part_floats, int *counters, hipStream_t s);
+// The same over the workspace layout of sp_attn_workspace_floats.
+hipError_t sp_launch_attn_wave_ws(const SpPlan &KP, const SpPlan &VP, const int *order, const SpAttnArgs &A,
+                                  const SpSeqTab &T, float *workspace, size_t ws_floats, hipStream_t s);
 hipError_t sp_launch_attn_f16(const unsigned short *k, const unsigned short *v,
                               long long head_stride, int n_kv, int n_q, int n_kvh, int hd,
                               float kq_scale, const float *q, float *scores, float *out,

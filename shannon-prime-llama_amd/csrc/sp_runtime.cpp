@@ -435,9 +435,6 @@ struct ShipPriv {
     float *ws = nullptr;
     size_t ws_floats = 0;
     int max_q = 0;
-    // batched (multi-sequence) attention workspace, grown on demand
-    float *seq_ws = nullptr;
-    size_t seq_ws_floats = 0;
     // K coefficient-order calibration: fp64 sums of the fed vectors' transforms
     bool calibrating = false;
     std::vector<double> csum, csum2;
@@ -545,7 +542,6 @@ extern "C" void sp_hip_cache_free(sp_hip_cache_t *cc) {
     ShipPriv *pv = (ShipPriv *)cc->priv;
     if (pv) {
         if (pv->ws) (void)hipFree(pv->ws);
-        if (pv->seq_ws) (void)hipFree(pv->seq_ws);
         if (pv->stage_d) (void)hipFree(pv->stage_d);
         if (pv->stage_h) (void)hipHostFree(pv->stage_h);
         delete pv;
@@ -895,6 +891,7 @@ int sp_attn_prepare(const sp_hip_cache_t *cc, int layer, int n_kv, const float *
     A.kpack = slot_ptr(cc, 0, layer, 0, 0);
     A.vpack = slot_ptr(cc, 1, layer, 0, 0);
     A.n_kv = n_kv;
+    A.start = 0;
     A.n_q = n_q;
     A.n_kvh = H;
     A.hd = cc->config.head_dim;
@@ -942,22 +939,11 @@ extern "C" int sp_hip_attn_decode_seqs(const sp_hip_cache_t *cc, int layer, int 
     if (!d_scores && !d_out) { set_err("attn seqs: no output"); return -1; }
     ShipPriv *pv = (ShipPriv *)cc->priv;
     const hipStream_t s = (hipStream_t)(stream ? stream : cc->stream);
-    // the one-position-per-lane layouts (hd 96 / hd 64): every sequence in one launch each of
-    // the query preparation, the split kernel and the combine
-    const char *off = getenv("SP_HIP_NO_LANE_ATTN");
-    int n_runs = (off && off[0] == '1') ? 0 : sp_attn_lane_runs(kp, vp, A, (size_t)1 << 40, n_seq);
-    for (int i = 0; i < n_seq && n_runs > 0; i++)  // the lane kernel's dword-aligned record bases, per sequence
-        if (((long long)T.start[i] * A.kB) % 4 || ((long long)T.start[i] * A.vB) % 4) n_runs = 0;
-    if (n_runs > 0) {
-        const size_t rows = (size_t)n_seq * n_q;
-        if (!grow_ws(&pv->seq_ws, &pv->seq_ws_floats, rows * A.hd + rows * n_runs * (A.hd + 2), s,
-                     "attn seqs workspace")) return -1;
-        return hip_ok(sp_launch_attn_lane_seqs(kp, vp, cc->d_mobius_order, A, T, pv->seq_ws, pv->seq_ws_floats, n_runs, s),
-                      "attn seqs") ? 0 : -1;
-    }
-    // otherwise one single-sequence launch sequence per sequence (the matrix-core kernel
-    // merges its partials inside its own launch), each over its range of records
     if (n_q > pv->max_q) { set_err("attn seqs: n_q %d > %d", n_q, pv->max_q); return -1; }
+    // the matrix-core layouts: every sequence in one launch, in the cache's own workspace
+    const hipError_t we = sp_launch_attn_wave_ws(kp, vp, cc->d_mobius_order, A, T, pv->ws, pv->ws_floats, s);
+    if (we != hipErrorNotSupported) return hip_ok(we, "attn seqs") ? 0 : -1;
+    // otherwise one single-sequence launch sequence per sequence, each over its range of records
     for (int i = 0; i < n_seq; i++) {
         SpAttnArgs Ai = A;
         Ai.kpack += (long long)T.start[i] * A.kB;
