@@ -283,12 +283,23 @@ hipError_t sp_launch_sqfree_attn(const SpPlan &KP, const SpPlan &VP, const SpSqG
                                  const SpSqAttnArgs &A, const SpSeqTab &T, float *ws, size_t ws_floats, int n_runs,
                                  hipStream_t s);
 
-// one-vector-per-lane hier kernels for the default geometry at head_dim 256;
-// hipErrorNotSupported (nothing launched) when no specialization fits. src2/dst2:
+// one-vector-per-lane hier kernels for the default geometry at head_dim 256 (fp16 rows; the
+// listed decode fp32 rows too); hipErrorNotSupported (nothing launched) when no
+// specialization fits. src2/dst2:
 // an optional second side (V with K) encoded by the same launch.
 hipError_t sp_launch_hier_encode_lane(const SpPlan &P, const SpHierGeo &G, const void *src, int dtype, long long so,
                                       long long si, unsigned char *dst, long long dout, int n_outer, int n_inner,
                                       hipStream_t s, const void *src2 = nullptr, unsigned char *dst2 = nullptr);
+// The same geometry with each 64-vector tile split over the waves of a block
+// (sp_hier_split.hip): any record alignment; src2/dst2 as above, for both directions. Whether
+// it is the faster one for `tiles` tiles that the lane kernels take in `launches` launches.
+bool sp_hier_split_pays(int dtype, long long tiles, int launches);
+hipError_t sp_launch_hier_encode_split(const SpPlan &P, const SpHierGeo &G, const void *src, int dtype, long long so,
+                                       long long si, unsigned char *dst, long long dout, int n_outer, int n_inner,
+                                       hipStream_t s, const void *src2 = nullptr, unsigned char *dst2 = nullptr);
+hipError_t sp_launch_hier_decode_split(const SpPlan &P, const SpHierGeo &G, const unsigned char *src, long long so,
+                                       void *dst, int dtype, long long dout, long long din, int n_outer, int n_inner,
+                                       hipStream_t s, const unsigned char *src2 = nullptr, void *dst2 = nullptr);
 // cells (optional): listed positions, record and row at cells[i] (slack after the cache)
 hipError_t sp_launch_hier_decode_lane(const SpPlan &P, const SpHierGeo &G, const unsigned char *src, long long so,
                                       void *dst, int dtype, long long dout, long long din, int n_outer, int n_inner,
@@ -322,6 +333,9 @@ hipError_t sp_launch_hier_encode(const SpPlan &P, const SpHierGeo &G, const void
 hipError_t sp_launch_hier_encode_kv(const SpPlan &P, const SpHierGeo &G, const void *src_k, const void *src_v,
                                     int dtype, long long so, long long si, unsigned char *dst_k,
                                     unsigned char *dst_v, long long dout, int n_outer, int n_inner, hipStream_t s);
+hipError_t sp_launch_hier_decode_kv(const SpPlan &P, const SpHierGeo &G, const unsigned char *src_k,
+                                    const unsigned char *src_v, long long so, void *dst_k, void *dst_v, int dtype,
+                                    long long dout, long long din, int n_outer, int n_inner, hipStream_t s);
 hipError_t sp_launch_hier_decode(const SpPlan &P, const SpHierGeo &G, const unsigned char *src,
                                  long long so, void *dst, int dtype, long long dout, long long din,
                                  int n_outer, int n_inner, hipStream_t s, const int *cells = nullptr);

@@ -1558,6 +1558,13 @@ extern "C" int sp_hip_hier_read_layer(const sp_hip_hier_cache_t *hc, int layer, 
     const int H = hc->config.n_heads_kv, hd = hc->config.head_dim;
     if (row_stride < (long long)H * hd) { set_err("hier read_layer: row_stride"); return -1; }
     const SpHierGeo G = hier_geo(hc, layer * H);
+    if (d_k && d_v) {  // one launch for both sides, as for the writes
+        const long long rec0 = ((long long)layer * H * hc->max_seq_len + start_pos) * G.bytes;
+        return hip_ok(sp_launch_hier_decode_kv(((HierPriv *)hc->priv)->plan, G, hc->d_k_cache + rec0, hc->d_v_cache + rec0,
+                                               (long long)hc->max_seq_len * G.bytes, d_k, d_v, dtype, hd, row_stride, H,
+                                               n_tok, (hipStream_t)hc->stream),
+                      "hier read_layer") ? 0 : -1;
+    }
     for (int is_v = 0; is_v < 2; is_v++) {
         void *dst = is_v ? d_v : d_k;
         if (!dst) continue;

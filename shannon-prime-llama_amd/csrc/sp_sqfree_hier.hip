@@ -323,7 +323,13 @@ hipError_t sp_launch_hier_encode(const SpPlan &P, const SpHierGeo &G, const void
     if (n_outer <= 0 || n_inner <= 0) return hipSuccess;
     if (!sq_fits(P, G.pad, G.bytes)) return hipErrorInvalidValue;
     if (!getenv_lane_off_sq()) {
-        const hipError_t e = sp_launch_hier_encode_lane(P, G, src, dtype, so, si, dst, dout, n_outer, n_inner, s);
+        hipError_t e = hipErrorNotSupported;
+        if (sp_hier_split_pays(dtype, (long long)n_outer * ((n_inner + 63) / 64), 1))
+            e = sp_launch_hier_encode_split(P, G, src, dtype, so, si, dst, dout, n_outer, n_inner, s);
+        if (e == hipErrorNotSupported)
+            e = sp_launch_hier_encode_lane(P, G, src, dtype, so, si, dst, dout, n_outer, n_inner, s);
+        if (e == hipErrorNotSupported)
+            e = sp_launch_hier_encode_split(P, G, src, dtype, so, si, dst, dout, n_outer, n_inner, s);
         if (e != hipErrorNotSupported) return e;
     }
     const long long nv = (long long)n_outer * n_inner;
@@ -341,8 +347,11 @@ hipError_t sp_launch_hier_encode_kv(const SpPlan &P, const SpHierGeo &G, const v
     if (n_outer <= 0 || n_inner <= 0) return hipSuccess;
     if (!sq_fits(P, G.pad, G.bytes)) return hipErrorInvalidValue;
     if (!getenv_lane_off_sq()) {
-        const hipError_t e = sp_launch_hier_encode_lane(P, G, src_k, dtype, so, si, dst_k, dout, n_outer, n_inner, s,
-                                                        src_v, dst_v);
+        hipError_t e = hipErrorNotSupported;
+        if (sp_hier_split_pays(dtype, 2LL * n_outer * ((n_inner + 63) / 64), 1))
+            e = sp_launch_hier_encode_split(P, G, src_k, dtype, so, si, dst_k, dout, n_outer, n_inner, s, src_v, dst_v);
+        if (e == hipErrorNotSupported)
+            e = sp_launch_hier_encode_lane(P, G, src_k, dtype, so, si, dst_k, dout, n_outer, n_inner, s, src_v, dst_v);
         if (e != hipErrorNotSupported) return e;
     }
     const hipError_t e = sp_launch_hier_encode(P, G, src_k, dtype, so, si, dst_k, dout, n_outer, n_inner, s);
@@ -356,7 +365,13 @@ hipError_t sp_launch_hier_decode(const SpPlan &P, const SpHierGeo &G, const unsi
     if (n_outer <= 0 || n_inner <= 0) return hipSuccess;
     if (!sq_fits(P, G.pad, G.bytes)) return hipErrorInvalidValue;
     if (!getenv_lane_off_sq()) {
-        const hipError_t e = sp_launch_hier_decode_lane(P, G, src, so, dst, dtype, dout, din, n_outer, n_inner, s, cells);
+        hipError_t e = hipErrorNotSupported;
+        if (!cells && sp_hier_split_pays(dtype, (long long)n_outer * ((n_inner + 63) / 64), 1))
+            e = sp_launch_hier_decode_split(P, G, src, so, dst, dtype, dout, din, n_outer, n_inner, s);
+        if (e == hipErrorNotSupported)
+            e = sp_launch_hier_decode_lane(P, G, src, so, dst, dtype, dout, din, n_outer, n_inner, s, cells);
+        if (e == hipErrorNotSupported && !cells)
+            e = sp_launch_hier_decode_split(P, G, src, so, dst, dtype, dout, din, n_outer, n_inner, s);
         if (e != hipErrorNotSupported) return e;
     }
     const long long nv = (long long)n_outer * n_inner;
@@ -366,4 +381,19 @@ hipError_t sp_launch_hier_decode(const SpPlan &P, const SpHierGeo &G, const unsi
     else
         hipLaunchKernelGGL((k_hier_decode<SP_DT_F32>), grid, block, 0, s, P, G, src, so, dst, dout, din, n_outer, n_inner, cells);
     return hipGetLastError();
+}
+
+hipError_t sp_launch_hier_decode_kv(const SpPlan &P, const SpHierGeo &G, const unsigned char *src_k,
+                                    const unsigned char *src_v, long long so, void *dst_k, void *dst_v, int dtype,
+                                    long long dout, long long din, int n_outer, int n_inner, hipStream_t s) {
+    if (n_outer <= 0 || n_inner <= 0) return hipSuccess;
+    if (!sq_fits(P, G.pad, G.bytes)) return hipErrorInvalidValue;
+    if (!getenv_lane_off_sq() && sp_hier_split_pays(dtype, 2LL * n_outer * ((n_inner + 63) / 64), 2)) {
+        const hipError_t e =
+            sp_launch_hier_decode_split(P, G, src_k, so, dst_k, dtype, dout, din, n_outer, n_inner, s, src_v, dst_v);
+        if (e != hipErrorNotSupported) return e;
+    }
+    const hipError_t e = sp_launch_hier_decode(P, G, src_k, so, dst_k, dtype, dout, din, n_outer, n_inner, s);
+    if (e != hipSuccess) return e;
+    return sp_launch_hier_decode(P, G, src_v, so, dst_v, dtype, dout, din, n_outer, n_inner, s);
 }
