@@ -397,7 +397,8 @@ __device__ __forceinline__ float rcp_f16_scale(float s) {
 }
 
 // Band-quantize coefficients x[src_idx(r)], r in [0, LY::hd), into the record
-// bits [0, 8 * LY::total) of rec (which must start zeroed there):
+// bits [0, 8 * LY::total) of rec (whose LY::dwords words must start as zero, the
+// rest of the last one too: sums of codes out of range carry into it):
 // kernel_band_quantize_simple (shannon_prime_cuda.cu:131-204). fastv: every
 // coefficient is finite.
 //
@@ -436,10 +437,8 @@ __device__ __forceinline__ void quant_bands(const float (&x)[N], bool fastv, uin
         }
     }
     if (!ok) {
-        constexpr int TW = LY::total / 4, TB = LY::total % 4;
 #pragma unroll
-        for (int d = 0; d < TW; d++) rec[d] = 0u;
-        if (TB) rec[TW] &= ~((1u << (8 * TB)) - 1u);
+        for (int d = 0; d < LY::dwords; d++) rec[d] = 0u;
 #pragma unroll
         for (int b = 0; b < LY::nb; b++) {
             const int off = LY::off(b), sz = LY::sz(b), bits = LY::bits[b];

@@ -1,0 +1,116 @@
+"""Layer calls of the one-vector-per-lane codec kernels at record runs of every address class:
+even-sized records (26 to 76 bytes) from any cell of odd- and even-length slots, tile edges,
+rows of infinities and NaN; records and reconstructions bit for bit against the oracle, and
+nothing written outside the run."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+import oracle_py as O  # noqa: E402
+import sp_hip as S  # noqa: E402
+import workloads as W  # noqa: E402
+from gpu_util import d2h, dev, p  # noqa: E402
+from test_gpu_attn import say  # noqa: E402
+
+SHIP = [(64, [5, 4, 4], [5]), (64, [5, 5, 4, 3], [3]), (96, [5, 4, 4], [5]), (128, [5, 5, 4, 3], [3])]
+RUNS = [(1, 0), (1, 1), (63, 1), (64, 2), (65, 3), (130, 1)]
+
+
+def _inputs(hd, H, n, f32):
+    kv = W.cfg1_kv(n_heads=H, n_pos=n, hd=hd, seed=hd + n)
+    for x in kv:
+        x[0, n // 2, 7] = np.inf
+        x[H - 1, n - 1, hd - 1] = np.nan
+        x[H - 1, 0, :] = 0
+    xs = [x.astype(np.float32) * np.float32(1 + 2.0 ** -12) if f32 else x for x in kv]
+    return xs, [dev((r if f32 else r.view(np.uint16)).transpose(1, 0, 2).reshape(n, H * hd)) for r in xs]
+
+
+def _records(cc, B, H, ms):
+    torch.cuda.synchronize()
+    return [d2h(q, H * ms * b).reshape(H, ms, b) for q, b in zip((cc.c.d_k_cache, cc.c.d_v_cache), B)]
+
+
+def _same(got, ref, f32):
+    bits = np.uint32 if f32 else np.uint16
+    nan = np.isnan(ref)
+    np.testing.assert_array_equal(np.isnan(got), nan)
+    np.testing.assert_array_equal(np.where(nan, 0, got).view(bits), np.where(nan, 0, ref).view(bits))
+
+
+def _check(cc, write, read, compress, decompress, B, hd, n, start, f32):
+    H, ms = 2, start + n + 3
+    xs, t = _inputs(hd, H, n, f32)
+    dt = S.DTYPE_F32 if f32 else S.DTYPE_F16
+    S.check(write(cc.ref, 0, start, n, p(t[0]), p(t[1]), H * hd, dt))
+    out = [torch.full((n, H, hd), 7.0, dtype=torch.float32 if f32 else torch.float16, device="cuda") for _ in range(2)]
+    S.check(read(cc, start, n, p(out[0]), p(out[1]), H * hd, dt))
+    both = _records(cc, B, H, ms)
+    for side in range(2):
+        for h in range(H):
+            ref = compress[side](xs[side][h])
+            np.testing.assert_array_equal(both[side][h, start:start + n], ref)
+            assert not both[side][h, :start].any() and not both[side][h, start + n:].any()
+            rec = decompress[side](ref)
+            _same(out[side][:, h].cpu().numpy(), rec if f32 else rec.astype(np.float16), f32)
+    # one side alone gives what both gave
+    alone = [torch.full_like(o, 7.0) for o in out]
+    for side in range(2):
+        a = [None, None]
+        a[side] = p(t[side])
+        S.check(write(cc.ref, 0, start, n, a[0], a[1], H * hd, dt))
+        a[side] = p(alone[side])
+        S.check(read(cc, start, n, a[0], a[1], H * hd, dt))
+    for b, c in zip(both, _records(cc, B, H, ms)):
+        np.testing.assert_array_equal(b, c)
+    for o, c in zip(out, alone):
+        _same(c.cpu().numpy(), o.cpu().numpy(), f32)
+    cc.free()
+
+
+@pytest.mark.parametrize("f32", [False, True])
+@pytest.mark.parametrize("n,start", RUNS)
+@pytest.mark.parametrize("hd,kb,vb", SHIP)
+def test_ship_layer(hd, kb, vb, n, start, f32):
+    say(f"lane cells ship hd={hd} k={kb} v={vb} n={n} start={start} f32={f32}")
+    cc = S.ShipCache(S.config(hd, 1, 2, k_bits=kb, v_bits=vb), start + n + 3,
+                     stream=torch.cuda.current_stream().cuda_stream)
+    bcs, orders = [O.band_config(hd, kb), O.band_config(hd, vb)], [O.mobius_order(hd), None]
+
+    def comp(s):
+        return lambda x: O.ship_compress_f32(x, bcs[s], orders[s]) if f32 else \
+            O.ship_compress_f16(x.view(np.uint16), bcs[s], orders[s])
+
+    def dec(s):
+        return lambda r: O.ship_decompress_f32(r, bcs[s], orders[s])
+
+    def read(c, start, n, k, v, stride, dt):
+        return S.lib().sp_hip_read_layer(c.ref, 0, start, n, k, v, stride, dt, -1)
+
+    _check(cc, S.lib().sp_hip_write_layer, read, [comp(0), comp(1)], [dec(0), dec(1)],
+           [b.total_bytes for b in bcs], hd, n, start, f32)
+
+
+@pytest.mark.parametrize("n,start", RUNS)
+@pytest.mark.parametrize("v_bits", [[5, 4, 4, 4, 5], [3]])
+def test_sqfree_layer(v_bits, n, start):
+    hd, k_bits = 128, [5, 4, 4, 4, 5]
+    say(f"lane cells sqfree v={v_bits} n={n} start={start}")
+    cc = S.SqfreeCache(S.config(hd, 1, 2, k_bits=k_bits, v_bits=v_bits), start + n + 3, rbits=3, spinor=True, sk_k=115,
+                       stream=torch.cuda.current_stream().cuda_stream)
+    km = O.Knight(154, 115)
+    bcs = [O.band_config(115, k_bits), O.band_config(115, v_bits)]
+
+    def comp(s):
+        return lambda x: O.sqfree_compress_f16(x.view(np.uint16), hd, km, bcs[s], 3, True)
+
+    def dec(s):
+        return lambda r: O.sqfree_decompress_f32(r, hd, km, bcs[s], 3, True)
+
+    def read(c, start, n, k, v, stride, dt):
+        return S.lib().sp_hip_sqfree_read_layer(c.ref, 0, start, n, k, v, stride, dt)
+
+    _check(cc, S.lib().sp_hip_sqfree_write_layer, read, [comp(0), comp(1)], [dec(0), dec(1)],
+           [cc.c.bytes_per_pos_k, cc.c.bytes_per_pos_v], hd, n, start, False)
