@@ -282,6 +282,10 @@ using K128 = Layout<128, 5, 5, 4, 3>;
 using V128 = Layout<128, 3>;
 using K64 = Layout<64, 5, 5, 4, 3>;
 using V64 = Layout<64, 5>;
+// head_dim 64 with the bridge's K bands, and with the shipping V band (8 heads x 1999
+// fp32 tokens from an odd cell, K: 27 us on the general kernel, 6 here)
+using K64b = Layout<64, 5, 4, 4>;
+using V64s = Layout<64, 3>;
 // Phi-3-mini-shaped hd 96 (Vilenkin 2^5 * 3) with the bridge's defaults, K 5/4/4 and V 5
 // (shannon_prime_llama.c:240-248)
 using K96 = Layout<96, 5, 4, 4>;
@@ -373,6 +377,7 @@ hipError_t enc_dispatch(const SpPlan &P, bool mob, const void *src, long long so
 #define SP_TRY(LY, MOB) \
     if (layout_matches<LY>(P)) return enc_launch<LY, DT, MOB>(P, mob, src, so, si, dst, dout, n_outer, n_inner, s);
     SP_TRY(K128, true) SP_TRY(V128, false) SP_TRY(K64, true) SP_TRY(V64, false) SP_TRY(K96, true) SP_TRY(V96, false) SP_TRY(V256, false)
+    SP_TRY(K64b, true) SP_TRY(V64s, false)
 #undef SP_TRY
     return hipErrorNotSupported;
 }
@@ -383,6 +388,7 @@ hipError_t dec_dispatch(const SpPlan &P, bool mob, const unsigned char *src, lon
 #define SP_TRY(LY, MOB) \
     if (layout_matches<LY>(P)) return dec_launch<LY, DT, MOB>(P, mob, src, so, dst, dout, din, n_outer, n_inner, s);
     SP_TRY(K128, true) SP_TRY(V128, false) SP_TRY(K64, true) SP_TRY(V64, false) SP_TRY(K96, true) SP_TRY(V96, false) SP_TRY(K256, true) SP_TRY(V256, false)
+    SP_TRY(K64b, true) SP_TRY(V64s, false)
 #undef SP_TRY
     return hipErrorNotSupported;
 }
@@ -391,12 +397,18 @@ hipError_t dec_dispatch(const SpPlan &P, bool mob, const unsigned char *src, lon
 
 // Returns hipErrorNotSupported (nothing launched) when no specialization fits:
 // the caller then uses the general kernels.
+//
+// Records may start at any even address: the record runs move as 16-byte buffer
+// accesses, which the hardware takes at any alignment, and one 2-byte access per
+// lane for the rest of an even-sized record run. So a run from an odd cell of 42-,
+// 50-, 58- or 62-byte records stays here (8 heads x 2048 tokens of head_dim 96 from
+// cell 1: encode 44 us on the general kernel, 7.9 here; 7.7 from cell 0).
 hipError_t sp_launch_ship_encode_lane(const SpPlan &P, bool default_order, const void *src, int dtype,
                                       long long so, long long si, unsigned char *dst, long long dout,
                                       int n_outer, int n_inner, hipStream_t s) {
     const int esz = dtype == SP_DT_F16 ? 2 : 4;
     if (((uintptr_t)src % 16) || ((so * esz) % 16) || ((si * esz) % 16)) return hipErrorNotSupported;
-    if (((uintptr_t)dst % 4) || (dout % 4)) return hipErrorNotSupported;
+    if (((uintptr_t)dst % 2) || (dout % 2)) return hipErrorNotSupported;
     if (dtype == SP_DT_F16) return enc_dispatch<SP_DT_F16>(P, default_order, src, so, si, dst, dout, n_outer, n_inner, s);
     return enc_dispatch<SP_DT_F32>(P, default_order, src, so, si, dst, dout, n_outer, n_inner, s);
 }
@@ -406,7 +418,7 @@ hipError_t sp_launch_ship_decode_lane(const SpPlan &P, bool default_order, const
                                       int n_outer, int n_inner, hipStream_t s) {
     const int esz = dtype == SP_DT_F16 ? 2 : 4;
     if (((uintptr_t)dst % 16) || ((dout * esz) % 16) || ((din * esz) % 16)) return hipErrorNotSupported;
-    if (((uintptr_t)src % 4) || (so % 4)) return hipErrorNotSupported;
+    if (((uintptr_t)src % 2) || (so % 2)) return hipErrorNotSupported;
     if (dtype == SP_DT_F16) return dec_dispatch<SP_DT_F16>(P, default_order, src, so, dst, dout, din, n_outer, n_inner, s);
     return dec_dispatch<SP_DT_F32>(P, default_order, src, so, dst, dout, din, n_outer, n_inner, s);
 }

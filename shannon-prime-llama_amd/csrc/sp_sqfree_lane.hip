@@ -286,13 +286,14 @@ hipError_t sp_launch_sqfree_decode_lane_cells(const SpPlan &P, const SpSqGeo &G,
 
 // Returns hipErrorNotSupported (nothing launched) when the geometry or the
 // operand alignment has no lane specialization: the caller then uses the
-// one-vector-per-wave kernels.
+// one-vector-per-wave kernels. Records may start at any even address (8 heads x
+// 2048 tokens of the 70-byte V records from cell 1: encode 85 us there, 18.3 here).
 hipError_t sp_launch_sqfree_encode_lane(const SpPlan &P, const SpSqGeo &G, const void *src, int dtype, long long so,
                                         long long si, unsigned char *dst, long long dout, int n_outer, int n_inner,
                                         hipStream_t s) {
     const int esz = dtype == SP_DT_F16 ? 2 : 4;
     if (((uintptr_t)src % 16) || ((so * esz) % 16) || ((si * esz) % 16)) return hipErrorNotSupported;
-    if (((uintptr_t)dst % 4) || (dout % 4)) return hipErrorNotSupported;
+    if (((uintptr_t)dst % 2) || (dout % 2)) return hipErrorNotSupported;
     if (sq_geometry_matches<77, SkelL77>(P, G))
         return dtype == SP_DT_F16 ? sq_enc_launch<SP_DT_F16, 77, SkelL77>(P, src, so, si, dst, dout, n_outer, n_inner, s)
                                   : sq_enc_launch<SP_DT_F32, 77, SkelL77>(P, src, so, si, dst, dout, n_outer, n_inner, s);
@@ -310,7 +311,7 @@ hipError_t sp_launch_sqfree_decode_lane(const SpPlan &P, const SpSqGeo &G, const
                                         int n_inner, hipStream_t s) {
     const int esz = dtype == SP_DT_F16 ? 2 : 4;
     if (((uintptr_t)dst % 16) || ((dout * esz) % 16) || ((din * esz) % 16)) return hipErrorNotSupported;
-    if (((uintptr_t)src % 4) || (so % 4)) return hipErrorNotSupported;
+    if (((uintptr_t)src % 2) || (so % 2)) return hipErrorNotSupported;
     if (sq_geometry_matches<77, SkelL77>(P, G))
         return dtype == SP_DT_F16 ? sq_dec_launch<SP_DT_F16, 77, SkelL77>(P, src, so, dst, dout, din, n_outer, n_inner, s)
                                   : sq_dec_launch<SP_DT_F32, 77, SkelL77>(P, src, so, dst, dout, din, n_outer, n_inner, s);
