@@ -160,6 +160,32 @@ hipError_t sp_launch_ship_encode(const SpPlan &P, const int *order, const void *
 hipError_t sp_launch_ship_decode(const SpPlan &P, const int *order, const unsigned char *src,
                                  long long so, void *dst, int dtype, long long dout, long long din,
                                  int n_outer, int n_inner, hipStream_t s);
+// K and V of one call (the same rows, strides and counts), in one launch where the
+// chip would be idle for half of each
+hipError_t sp_launch_ship_encode_kv(const SpPlan &KP, const int *korder, const SpPlan &VP, const void *src_k,
+                                    const void *src_v, int dtype, long long so, long long si, unsigned char *dst_k,
+                                    unsigned char *dst_v, long long dout_k, long long dout_v, int n_outer, int n_inner,
+                                    hipStream_t s);
+hipError_t sp_launch_ship_decode_kv(const SpPlan &KP, const int *korder, const SpPlan &VP, const unsigned char *src_k,
+                                    const unsigned char *src_v, long long so_k, long long so_v, void *dst_k,
+                                    void *dst_v, int dtype, long long dout, long long din, int n_outer, int n_inner,
+                                    hipStream_t s);
+// Whether no element of side k's rows (row (o, i) of hd elements at o*dout + i*din)
+// is an element of side v's: the two sides of a read may then be written in any order.
+// Exact for one outer row per hd columns of a token row (dout == hd: layer calls) and
+// for whole extents; true only where that is certain.
+inline bool sp_kv_rows_disjoint(const void *k, const void *v, int dtype, int hd, long long dout, long long din,
+                                int n_outer, int n_inner) {
+    const long long esz = dtype == SP_DT_F16 ? 2 : 4;
+    const unsigned long long a = (unsigned long long)(uintptr_t)k, b = (unsigned long long)(uintptr_t)v;
+    const unsigned long long d = a < b ? b - a : a - b;
+    if (dout < 0 || din < 0) return false;
+    const unsigned long long ext = (unsigned long long)(((n_outer - 1) * dout + (n_inner - 1) * din + hd) * esz);
+    if (d >= ext) return true;
+    if (dout != hd || din < (long long)n_outer * hd) return false;
+    const unsigned long long w = (unsigned long long)n_outer * hd * esz, st = (unsigned long long)din * esz, r = d % st;
+    return r >= w && st - r >= w;
+}
 hipError_t sp_launch_ship_encode_generic(const SpPlan &P, const int *order, const void *src,
                                          int dtype, long long so, long long si, unsigned char *dst,
                                          long long dout, int n_outer, int n_inner, hipStream_t s);
@@ -176,6 +202,14 @@ hipError_t sp_launch_ship_encode_lane(const SpPlan &P, bool default_order, const
 hipError_t sp_launch_ship_decode_lane(const SpPlan &P, bool default_order, const unsigned char *src,
                                       long long so, void *dst, int dtype, long long dout, long long din,
                                       int n_outer, int n_inner, hipStream_t s);
+hipError_t sp_launch_ship_encode_lane_kv(const SpPlan &KP, const SpPlan &VP, const void *src_k, const void *src_v,
+                                         int dtype, long long so, long long si, unsigned char *dst_k,
+                                         unsigned char *dst_v, long long dout_k, long long dout_v, int n_outer,
+                                         int n_inner, hipStream_t s);
+hipError_t sp_launch_ship_decode_lane_kv(const SpPlan &KP, const SpPlan &VP, const unsigned char *src_k,
+                                         const unsigned char *src_v, long long so_k, long long so_v, void *dst_k,
+                                         void *dst_v, int dtype, long long dout, long long din, int n_outer,
+                                         int n_inner, hipStream_t s);
 // in-place compress + decompress of every head's vectors at n_cells cache cells
 // (element (c, h, d) at c*cs + (h*hd + d)*es of x; records at rec_base +
 // h*rec_head_stride + c*B); hipErrorNotSupported when no specialization fits
@@ -317,6 +351,23 @@ hipError_t sp_launch_sqfree_decode_lane(const SpPlan &P, const SpSqGeo &G, const
 hipError_t sp_launch_sqfree_decode_lane_cells(const SpPlan &P, const SpSqGeo &G, const unsigned char *src,
                                               long long so, void *dst, int dtype, long long dout, long long din,
                                               int n_outer, int n_inner, const int *cells, hipStream_t s);
+// both sides in one launch (GK, GV differ in record bytes only)
+hipError_t sp_launch_sqfree_encode_lane_kv(const SpPlan &KP, const SpPlan &VP, const SpSqGeo &GK, const SpSqGeo &GV,
+                                           const void *src_k, const void *src_v, int dtype, long long so, long long si,
+                                           unsigned char *dst_k, unsigned char *dst_v, long long dout_k,
+                                           long long dout_v, int n_outer, int n_inner, hipStream_t s);
+hipError_t sp_launch_sqfree_decode_lane_kv(const SpPlan &KP, const SpPlan &VP, const SpSqGeo &GK, const SpSqGeo &GV,
+                                           const unsigned char *src_k, const unsigned char *src_v, long long so_k,
+                                           long long so_v, void *dst_k, void *dst_v, int dtype, long long dout,
+                                           long long din, int n_outer, int n_inner, hipStream_t s);
+hipError_t sp_launch_sqfree_encode_kv(const SpPlan &KP, const SpPlan &VP, const SpSqGeo &GK, const SpSqGeo &GV,
+                                      const void *src_k, const void *src_v, int dtype, long long so, long long si,
+                                      unsigned char *dst_k, unsigned char *dst_v, long long dout_k, long long dout_v,
+                                      int n_outer, int n_inner, hipStream_t s);
+hipError_t sp_launch_sqfree_decode_kv(const SpPlan &KP, const SpPlan &VP, const SpSqGeo &GK, const SpSqGeo &GV,
+                                      const unsigned char *src_k, const unsigned char *src_v, long long so_k,
+                                      long long so_v, void *dst_k, void *dst_v, int dtype, long long dout,
+                                      long long din, int n_outer, int n_inner, hipStream_t s);
 hipError_t sp_launch_sqfree_encode(const SpPlan &P, const SpSqGeo &G, const void *src, int dtype,
                                    long long so, long long si, unsigned char *dst, long long dout,
                                    int n_outer, int n_inner, hipStream_t s);

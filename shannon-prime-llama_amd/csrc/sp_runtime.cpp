@@ -606,6 +606,12 @@ extern "C" int sp_hip_write_layer(sp_hip_cache_t *cc, int layer, int start_pos, 
     if (row_stride < (long long)H * hd) { set_err("write_layer: row_stride"); return -1; }
     ShipPriv *pv = (ShipPriv *)cc->priv;
     hipStream_t s = (hipStream_t)cc->stream;
+    if (d_k && d_v)
+        return hip_ok(sp_launch_ship_encode_kv(pv->kplan, cc->d_mobius_order, pv->vplan, d_k, d_v, dtype, hd, row_stride,
+                                               slot_ptr(cc, 0, layer, 0, start_pos), slot_ptr(cc, 1, layer, 0, start_pos),
+                                               (long long)cc->max_seq_len * cc->k_bands.total_bytes,
+                                               (long long)cc->max_seq_len * cc->v_bands.total_bytes, H, n_tok, s),
+                      "write_layer") ? 0 : -1;
     if (d_k && !hip_ok(sp_launch_ship_encode(pv->kplan, cc->d_mobius_order, d_k, dtype, hd, row_stride,
                                              slot_ptr(cc, 0, layer, 0, start_pos),
                                              (long long)cc->max_seq_len * cc->k_bands.total_bytes, H,
@@ -629,6 +635,13 @@ extern "C" int sp_hip_read_layer(const sp_hip_cache_t *cc, int layer, int start_
         if (max_bands < kp.n_bands) kp.max_bands = max_bands;
         if (max_bands < vp.n_bands) vp.max_bands = max_bands;
     }
+    if (d_k && d_v)
+        return hip_ok(sp_launch_ship_decode_kv(kp, cc->d_mobius_order, vp, slot_ptr(cc, 0, layer, 0, start_pos),
+                                               slot_ptr(cc, 1, layer, 0, start_pos),
+                                               (long long)cc->max_seq_len * cc->k_bands.total_bytes,
+                                               (long long)cc->max_seq_len * cc->v_bands.total_bytes, d_k, d_v, dtype, hd,
+                                               row_stride, H, n_tok, s),
+                      "read_layer") ? 0 : -1;
     if (d_k && !hip_ok(sp_launch_ship_decode(kp, cc->d_mobius_order, slot_ptr(cc, 0, layer, 0, start_pos),
                                              (long long)cc->max_seq_len * cc->k_bands.total_bytes, d_k,
                                              dtype, hd, row_stride, H, n_tok, s), "read_layer K")) return -1;
@@ -795,6 +808,13 @@ extern "C" int sp_hip_write_all(sp_hip_cache_t *cc, int start_pos, int n_pos, co
     const int n_slots = cc->config.n_layers * cc->config.n_heads_kv, hd = cc->config.head_dim;
     ShipPriv *pv = (ShipPriv *)cc->priv;
     hipStream_t s = (hipStream_t)cc->stream;
+    if (d_k && d_v)
+        return hip_ok(sp_launch_ship_encode_kv(pv->kplan, cc->d_mobius_order, pv->vplan, d_k, d_v, dtype,
+                                               (long long)n_pos * hd, hd, slot_ptr(cc, 0, 0, 0, start_pos),
+                                               slot_ptr(cc, 1, 0, 0, start_pos),
+                                               (long long)cc->max_seq_len * cc->k_bands.total_bytes,
+                                               (long long)cc->max_seq_len * cc->v_bands.total_bytes, n_slots, n_pos, s),
+                      "write_all") ? 0 : -1;
     if (d_k && !hip_ok(sp_launch_ship_encode(pv->kplan, cc->d_mobius_order, d_k, dtype, (long long)n_pos * hd, hd,
                                              slot_ptr(cc, 0, 0, 0, start_pos),
                                              (long long)cc->max_seq_len * cc->k_bands.total_bytes, n_slots,
@@ -817,6 +837,13 @@ extern "C" int sp_hip_read_all(const sp_hip_cache_t *cc, int start_pos, int n_po
         if (max_bands < kp.n_bands) kp.max_bands = max_bands;
         if (max_bands < vp.n_bands) vp.max_bands = max_bands;
     }
+    if (d_k && d_v)
+        return hip_ok(sp_launch_ship_decode_kv(kp, cc->d_mobius_order, vp, slot_ptr(cc, 0, 0, 0, start_pos),
+                                               slot_ptr(cc, 1, 0, 0, start_pos),
+                                               (long long)cc->max_seq_len * cc->k_bands.total_bytes,
+                                               (long long)cc->max_seq_len * cc->v_bands.total_bytes, d_k, d_v, dtype,
+                                               (long long)n_pos * hd, hd, n_slots, n_pos, s),
+                      "read_all") ? 0 : -1;
     if (d_k && !hip_ok(sp_launch_ship_decode(kp, cc->d_mobius_order, slot_ptr(cc, 0, 0, 0, start_pos),
                                              (long long)cc->max_seq_len * cc->k_bands.total_bytes, d_k,
                                              dtype, (long long)n_pos * hd, hd, n_slots, n_pos, s), "read_all K")) return -1;
@@ -1197,6 +1224,14 @@ extern "C" int sp_hip_sqfree_write_layer(sp_hip_sqfree_cache_t *cc, int layer, i
     const int H = cc->config.n_heads_kv, hd = cc->config.head_dim;
     if (row_stride < (long long)H * hd) { set_err("sqfree write_layer: row_stride"); return -1; }
     SqPriv *pv = (SqPriv *)cc->priv;
+    if (d_k && d_v) {
+        const SpSqGeo GK = sq_geo(cc, 0), GV = sq_geo(cc, 1);
+        const long long pos0 = (long long)layer * H * cc->max_seq_len + start_pos, ms = cc->max_seq_len;
+        return hip_ok(sp_launch_sqfree_encode_kv(pv->kplan, pv->vplan, GK, GV, d_k, d_v, dtype, hd, row_stride,
+                                                 cc->d_k_cache + pos0 * GK.bytes, cc->d_v_cache + pos0 * GV.bytes,
+                                                 ms * GK.bytes, ms * GV.bytes, H, n_tok, (hipStream_t)cc->stream),
+                      "sqfree write_layer") ? 0 : -1;
+    }
     for (int is_v = 0; is_v < 2; is_v++) {
         const void *src = is_v ? d_v : d_k;
         if (!src) continue;
@@ -1216,6 +1251,14 @@ extern "C" int sp_hip_sqfree_read_layer(const sp_hip_sqfree_cache_t *cc, int lay
     const int H = cc->config.n_heads_kv, hd = cc->config.head_dim;
     if (row_stride < (long long)H * hd) { set_err("sqfree read_layer: row_stride"); return -1; }
     SqPriv *pv = (SqPriv *)cc->priv;
+    if (d_k && d_v) {
+        const SpSqGeo GK = sq_geo(cc, 0), GV = sq_geo(cc, 1);
+        const long long pos0 = (long long)layer * H * cc->max_seq_len + start_pos, ms = cc->max_seq_len;
+        return hip_ok(sp_launch_sqfree_decode_kv(pv->kplan, pv->vplan, GK, GV, cc->d_k_cache + pos0 * GK.bytes,
+                                                 cc->d_v_cache + pos0 * GV.bytes, ms * GK.bytes, ms * GV.bytes, d_k, d_v,
+                                                 dtype, hd, row_stride, H, n_tok, (hipStream_t)cc->stream),
+                      "sqfree read_layer") ? 0 : -1;
+    }
     for (int is_v = 0; is_v < 2; is_v++) {
         void *dst = is_v ? d_v : d_k;
         if (!dst) continue;

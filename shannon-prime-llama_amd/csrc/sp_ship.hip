@@ -687,6 +687,40 @@ hipError_t sp_launch_ship_decode(const SpPlan &P, const int *order, const unsign
     return hipGetLastError();
 }
 
+// K and V of one call in one launch where a merged kernel takes the pair
+// (sp_ship_lane.hip), else one after the other.
+hipError_t sp_launch_ship_encode_kv(const SpPlan &KP, const int *korder, const SpPlan &VP, const void *src_k,
+                                    const void *src_v, int dtype, long long so, long long si, unsigned char *dst_k,
+                                    unsigned char *dst_v, long long dout_k, long long dout_v, int n_outer, int n_inner,
+                                    hipStream_t s) {
+    if (n_outer <= 0 || n_inner <= 0) return hipSuccess;
+    if (!KP.skip_transform && !VP.skip_transform && korder && KP.order_default && !getenv_lane_off()) {
+        const hipError_t e = sp_launch_ship_encode_lane_kv(KP, VP, src_k, src_v, dtype, so, si, dst_k, dst_v, dout_k,
+                                                           dout_v, n_outer, n_inner, s);
+        if (e != hipErrorNotSupported) return e;
+    }
+    const hipError_t e = sp_launch_ship_encode(KP, korder, src_k, dtype, so, si, dst_k, dout_k, n_outer, n_inner, s);
+    if (e != hipSuccess) return e;
+    return sp_launch_ship_encode(VP, nullptr, src_v, dtype, so, si, dst_v, dout_v, n_outer, n_inner, s);
+}
+
+hipError_t sp_launch_ship_decode_kv(const SpPlan &KP, const int *korder, const SpPlan &VP, const unsigned char *src_k,
+                                    const unsigned char *src_v, long long so_k, long long so_v, void *dst_k,
+                                    void *dst_v, int dtype, long long dout, long long din, int n_outer, int n_inner,
+                                    hipStream_t s) {
+    if (n_outer <= 0 || n_inner <= 0) return hipSuccess;
+    // two sides that share bytes (one buffer for both, say) keep their order
+    if (!KP.skip_transform && !VP.skip_transform && korder && KP.order_default && !getenv_lane_off() &&
+        sp_kv_rows_disjoint(dst_k, dst_v, dtype, KP.hd, dout, din, n_outer, n_inner)) {
+        const hipError_t e = sp_launch_ship_decode_lane_kv(KP, VP, src_k, src_v, so_k, so_v, dst_k, dst_v, dtype, dout,
+                                                           din, n_outer, n_inner, s);
+        if (e != hipErrorNotSupported) return e;
+    }
+    const hipError_t e = sp_launch_ship_decode(KP, korder, src_k, so_k, dst_k, dtype, dout, din, n_outer, n_inner, s);
+    if (e != hipSuccess) return e;
+    return sp_launch_ship_decode(VP, nullptr, src_v, so_v, dst_v, dtype, dout, din, n_outer, n_inner, s);
+}
+
 // Generic-only variants (used by tests to cross-check both kernel families).
 hipError_t sp_launch_ship_encode_generic(const SpPlan &P, const int *order, const void *src, int dtype,
                                          long long so, long long si, unsigned char *dst,

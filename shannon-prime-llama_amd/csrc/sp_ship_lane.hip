@@ -106,26 +106,49 @@ __device__ __forceinline__ void enc_tile(const uint4 (&in)[row_bytes<DT>(LY::hd)
 // Each single-wave block loads its tile with coalesced 16-byte loads and
 // transposes it through LDS; with no prefetch registers held across the
 // arithmetic, two waves fit per SIMD and one's loads overlap the other's work.
+// The record stage reuses the row buffer once the rows are in registers: 17 KB
+// per single-wave block lets two waves share each SIMD.
+template <class LY, int DT, int NORM, bool MOB>
+__device__ __forceinline__ void enc_tiles(const void *src, long long so, long long si, unsigned char *dst,
+                                          long long dout, const TileMap &M, int t, int step, int n_tiles,
+                                          const XfConst &K, unsigned char *rows) {
+    constexpr int RB = row_bytes<DT>(LY::hd), RP = RB + 16, CPR = RB / 16, B = LY::total, DW = LY::dwords;
+    static_assert(64 * B + 16 <= 64 * RP, "record stage must fit in the row buffer");
+    const int lane = threadIdx.x;
+    for (; t < n_tiles; t += step) {
+        uint4 in[CPR];
+        tile_rows_in<DT, LY::hd>(src, so, si, M, t, lane, rows, in);
+        uint32_t rec[DW];
+        enc_tile<LY, DT, NORM, MOB>(in, K, rec);
+        tile_records_out<B, 64 * RP>(rec, rows, dst, dout, M, t, lane);
+    }
+}
+
 template <class LY, int DT, int NORM, bool MOB>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DT == SP_DT_F16 ? 2 : 1)))
 k_ship_encode_lane(const void *__restrict__ src, long long so, long long si,
                    unsigned char *__restrict__ dst, long long dout, int n_inner, int tiles_per_outer,
                    int n_tiles, const XfConst K) {
-    constexpr int RB = row_bytes<DT>(LY::hd), RP = RB + 16, CPR = RB / 16, B = LY::total, DW = LY::dwords;
-    // the record stage reuses the row buffer once the rows are in registers:
-    // 17 KB per single-wave block lets two waves share each SIMD
-    __shared__ __attribute__((aligned(16))) unsigned char rows[64 * RP];
-    static_assert(64 * B + 16 <= 64 * RP, "record stage must fit in the row buffer");
-    unsigned char *const stage = rows;
-    const int lane = threadIdx.x;
+    __shared__ __attribute__((aligned(16))) unsigned char rows[64 * (row_bytes<DT>(LY::hd) + 16)];
+    enc_tiles<LY, DT, NORM, MOB>(src, so, si, dst, dout, TileMap{tiles_per_outer, n_inner}, blockIdx.x, gridDim.x,
+                                 n_tiles, K, rows);
+}
+
+// K and V of one call in one launch: the first half of the grid walks K's tiles,
+// the second half V's (the same tile counts and row strides).
+// One launch instead of two, and twice the tiles in flight, for calls whose tiles
+// leave the chip idle (kv_pays holds the figures).
+template <class LK, class LV, int DT>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DT == SP_DT_F16 ? 2 : 1)))
+k_ship_encode_lane_kv(const void *__restrict__ src_k, const void *__restrict__ src_v, long long so, long long si,
+                      unsigned char *__restrict__ dst_k, unsigned char *__restrict__ dst_v, long long dout_k,
+                      long long dout_v, int n_inner, int tiles_per_outer, int n_tiles, const XfConst K) {
+    static_assert(LK::hd == LV::hd, "both sides' rows go through the same stage");
+    __shared__ __attribute__((aligned(16))) unsigned char rows[64 * (row_bytes<DT>(LK::hd) + 16)];
+    const int nb = gridDim.x / 2, b = blockIdx.x;
     const TileMap M{tiles_per_outer, n_inner};
-    for (int t = blockIdx.x; t < n_tiles; t += gridDim.x) {
-        uint4 in[CPR];
-        tile_rows_in<DT, LY::hd>(src, so, si, M, t, lane, rows, in);
-        uint32_t rec[DW];
-        enc_tile<LY, DT, NORM, MOB>(in, K, rec);
-        tile_records_out<B, 64 * RP>(rec, stage, dst, dout, M, t, lane);
-    }
+    if (b < nb) enc_tiles<LK, DT, 0, true>(src_k, so, si, dst_k, dout_k, M, b, nb, n_tiles, K, rows);
+    else enc_tiles<LV, DT, 0, false>(src_v, so, si, dst_v, dout_v, M, b - nb, nb, n_tiles, K, rows);
 }
 
 // ---------------------------------------------------------------------------
@@ -160,28 +183,48 @@ __device__ __forceinline__ void dec_tile(const uint32_t (&rec)[LY::dwords], unsi
 // into registers, and are transposed through the LDS row stage (the records
 // are in registers before the stage is overwritten with output rows).
 template <class LY, int DT, int NORM, bool MOB, bool FULL>
-__global__ void __launch_bounds__(64)
-k_ship_decode_lane(const unsigned char *__restrict__ src, long long so, void *__restrict__ dst,
-                   long long dout, long long din, int n_inner, int tiles_per_outer, int n_tiles,
-                   const XfConst K, int max_bands) {
+__device__ __forceinline__ void dec_tiles(const unsigned char *src, long long so, void *dst, long long dout,
+                                          long long din, const TileMap &M, int t, int step, int n_tiles,
+                                          const XfConst &K, int max_bands, unsigned char *stage) {
     constexpr int RP = row_bytes<DT>(LY::hd) + 16, DW = LY::dwords, B = LY::total;
     constexpr int NCK = (64 * B / 16 + 63) / 64;
     static_assert(NCK * 1024 + 16 <= 64 * RP, "record tile must fit in the row stage");
-    __shared__ __attribute__((aligned(16))) unsigned char stage[64 * RP];
-    const int lane = threadIdx.x, G = gridDim.x;
-    const TileMap M{tiles_per_outer, n_inner};
+    const int lane = threadIdx.x;
     RecTile<LY> R;
-    int t = blockIdx.x;
     if (t >= n_tiles) return;
     rec_tile_load<LY>(R, src, so, M, t, n_tiles, lane);
-    for (; t < n_tiles; t += G) {
+    for (; t < n_tiles; t += step) {
         rec_tile_stage<LY>(R, stage, M, t, lane);
         __syncthreads();
-        rec_tile_load<LY>(R, src, so, M, t + G, n_tiles, lane);
+        rec_tile_load<LY>(R, src, so, M, t + step, n_tiles, lane);
         uint32_t rec[DW];
         rec_from_lds<LY>(rec, stage, lane);
         dec_tile<LY, DT, NORM, MOB, FULL>(rec, stage, dst, dout, din, M, t, lane, K, max_bands);
     }
+}
+
+template <class LY, int DT, int NORM, bool MOB, bool FULL>
+__global__ void __launch_bounds__(64)
+k_ship_decode_lane(const unsigned char *__restrict__ src, long long so, void *__restrict__ dst,
+                   long long dout, long long din, int n_inner, int tiles_per_outer, int n_tiles,
+                   const XfConst K, int max_bands) {
+    __shared__ __attribute__((aligned(16))) unsigned char stage[64 * (row_bytes<DT>(LY::hd) + 16)];
+    dec_tiles<LY, DT, NORM, MOB, FULL>(src, so, dst, dout, din, TileMap{tiles_per_outer, n_inner}, blockIdx.x,
+                                       gridDim.x, n_tiles, K, max_bands, stage);
+}
+
+// K and V of one call in one launch, every band, as k_ship_encode_lane_kv does it.
+template <class LK, class LV, int DT>
+__global__ void __launch_bounds__(64)
+k_ship_decode_lane_kv(const unsigned char *__restrict__ src_k, const unsigned char *__restrict__ src_v, long long so_k,
+                      long long so_v, void *__restrict__ dst_k, void *__restrict__ dst_v, long long dout, long long din,
+                      int n_inner, int tiles_per_outer, int n_tiles, const XfConst K) {
+    static_assert(LK::hd == LV::hd, "both sides' rows go through the same stage");
+    __shared__ __attribute__((aligned(16))) unsigned char stage[64 * (row_bytes<DT>(LK::hd) + 16)];
+    const int nb = gridDim.x / 2, b = blockIdx.x;
+    const TileMap M{tiles_per_outer, n_inner};
+    if (b < nb) dec_tiles<LK, DT, 0, true, true>(src_k, so_k, dst_k, dout, din, M, b, nb, n_tiles, K, LK::nb, stage);
+    else dec_tiles<LV, DT, 0, false, true>(src_v, so_v, dst_v, dout, din, M, b - nb, nb, n_tiles, K, LV::nb, stage);
 }
 
 // ---------------------------------------------------------------------------
@@ -358,6 +401,40 @@ hipError_t rt_launch(const SpPlan &P, bool mob, void *x, long long cs, long long
     return hipGetLastError();
 }
 
+// Both sides in one launch while all their tiles have a block of their own at once
+// (the persistent grid). Measured at 8 heads, both sides merged / one after the other,
+// us: head_dim 64 fp32 encode 6.0 / 11.0 at 256 tiles a side, 15.0 / 17.4 at 2048;
+// head_dim 128 fp16 encode 6.4 / 11.7 at 1, 8.6 / 14.2 at 512, 19.8 / 22.6 at 2048,
+// decode 8.4 / 13.7 at 512, 18.2 / 21.6 at 2048; head_dim 256 decode 16.2 / 24.9 at 512,
+// 56.3 / 64.5 at 2048. Past that both take the same time (41.0 / 40.8 at 4096), and
+// the large calls keep the kernels they were tuned on.
+long long kv_tiles(int n_outer, int n_inner) { return (long long)n_outer * ((n_inner + 63) / 64); }
+bool kv_pays(long long tiles) { return 2 * tiles <= persistent_blocks(); }
+
+template <class LK, class LV, int DT>
+hipError_t enc_kv_launch(const SpPlan &P, const void *src_k, const void *src_v, long long so, long long si,
+                         unsigned char *dst_k, unsigned char *dst_v, long long dout_k, long long dout_v, int n_outer,
+                         int n_inner, hipStream_t s) {
+    const int tpo = (n_inner + 63) / 64, n_tiles = (int)kv_tiles(n_outer, n_inner);
+    constexpr long long esz = DT == SP_DT_F16 ? 2 : 4;
+    if (si < 0 || 64 * si * esz + row_bytes<DT>(LK::hd) > 0x7fffffffLL) return hipErrorNotSupported;
+    hipLaunchKernelGGL((k_ship_encode_lane_kv<LK, LV, DT>), dim3(2 * n_tiles), dim3(64), 0, s, src_k, src_v, so, si,
+                       dst_k, dst_v, dout_k, dout_v, n_inner, tpo, n_tiles, xf_const(P));
+    return hipGetLastError();
+}
+
+template <class LK, class LV, int DT>
+hipError_t dec_kv_launch(const SpPlan &P, const unsigned char *src_k, const unsigned char *src_v, long long so_k,
+                         long long so_v, void *dst_k, void *dst_v, long long dout, long long din, int n_outer,
+                         int n_inner, hipStream_t s) {
+    const int tpo = (n_inner + 63) / 64, n_tiles = (int)kv_tiles(n_outer, n_inner);
+    constexpr long long esz = DT == SP_DT_F16 ? 2 : 4;
+    if (din < LK::hd || 64 * din * esz + row_bytes<DT>(LK::hd) > 0x7fffffffLL) return hipErrorNotSupported;
+    hipLaunchKernelGGL((k_ship_decode_lane_kv<LK, LV, DT>), dim3(2 * n_tiles), dim3(64), 0, s, src_k, src_v, so_k, so_v,
+                       dst_k, dst_v, dout, din, n_inner, tpo, n_tiles, xf_const(P));
+    return hipGetLastError();
+}
+
 template <int DT>
 hipError_t rt_dispatch(const SpPlan &P, bool mob, void *x, long long cs, long long es, const int *cells, int n_cells,
                        int max_seq, unsigned char *rec_base, long long rec_head_stride, int n_heads, int max_bands,
@@ -421,6 +498,51 @@ hipError_t sp_launch_ship_decode_lane(const SpPlan &P, bool default_order, const
     if (((uintptr_t)src % 2) || (so % 2)) return hipErrorNotSupported;
     if (dtype == SP_DT_F16) return dec_dispatch<SP_DT_F16>(P, default_order, src, so, dst, dout, din, n_outer, n_inner, s);
     return dec_dispatch<SP_DT_F32>(P, default_order, src, so, dst, dout, din, n_outer, n_inner, s);
+}
+
+// K and V in one launch (K in the default Mobius order, V in natural order, the
+// bridge's and the shipping band pairs); hipErrorNotSupported (nothing launched)
+// when the pair, the alignment or the size is not one the merged kernels take.
+hipError_t sp_launch_ship_encode_lane_kv(const SpPlan &KP, const SpPlan &VP, const void *src_k, const void *src_v,
+                                         int dtype, long long so, long long si, unsigned char *dst_k,
+                                         unsigned char *dst_v, long long dout_k, long long dout_v, int n_outer,
+                                         int n_inner, hipStream_t s) {
+    const int esz = dtype == SP_DT_F16 ? 2 : 4;
+    if (KP.norm != 0 || VP.norm != 0 || !kv_pays(kv_tiles(n_outer, n_inner))) return hipErrorNotSupported;
+    if (((uintptr_t)src_k % 16) || ((uintptr_t)src_v % 16) || ((so * esz) % 16) || ((si * esz) % 16) ||
+        ((uintptr_t)dst_k % 2) || ((uintptr_t)dst_v % 2) || (dout_k % 2) || (dout_v % 2))
+        return hipErrorNotSupported;
+#define SP_TRY(LK, LV)                                                                                              \
+    if (layout_matches<LK>(KP) && layout_matches<LV>(VP))                                                           \
+        return dtype == SP_DT_F16 ? enc_kv_launch<LK, LV, SP_DT_F16>(KP, src_k, src_v, so, si, dst_k, dst_v, dout_k, \
+                                                                     dout_v, n_outer, n_inner, s)                   \
+                                  : enc_kv_launch<LK, LV, SP_DT_F32>(KP, src_k, src_v, so, si, dst_k, dst_v, dout_k, \
+                                                                     dout_v, n_outer, n_inner, s);
+    SP_TRY(K128, V128) SP_TRY(K64b, V64) SP_TRY(K64, V64s) SP_TRY(K96, V96)
+#undef SP_TRY
+    return hipErrorNotSupported;
+}
+
+hipError_t sp_launch_ship_decode_lane_kv(const SpPlan &KP, const SpPlan &VP, const unsigned char *src_k,
+                                         const unsigned char *src_v, long long so_k, long long so_v, void *dst_k,
+                                         void *dst_v, int dtype, long long dout, long long din, int n_outer,
+                                         int n_inner, hipStream_t s) {
+    const int esz = dtype == SP_DT_F16 ? 2 : 4;
+    if (KP.norm != 0 || VP.norm != 0 || !kv_pays(kv_tiles(n_outer, n_inner))) return hipErrorNotSupported;
+    if ((KP.max_bands >= 0 && KP.max_bands < KP.n_bands) || (VP.max_bands >= 0 && VP.max_bands < VP.n_bands))
+        return hipErrorNotSupported;
+    if (((uintptr_t)dst_k % 16) || ((uintptr_t)dst_v % 16) || ((dout * esz) % 16) || ((din * esz) % 16) ||
+        ((uintptr_t)src_k % 2) || ((uintptr_t)src_v % 2) || (so_k % 2) || (so_v % 2))
+        return hipErrorNotSupported;
+#define SP_TRY(LK, LV)                                                                                              \
+    if (layout_matches<LK>(KP) && layout_matches<LV>(VP))                                                           \
+        return dtype == SP_DT_F16 ? dec_kv_launch<LK, LV, SP_DT_F16>(KP, src_k, src_v, so_k, so_v, dst_k, dst_v, dout, \
+                                                                     din, n_outer, n_inner, s)                      \
+                                  : dec_kv_launch<LK, LV, SP_DT_F32>(KP, src_k, src_v, so_k, so_v, dst_k, dst_v, dout, \
+                                                                     din, n_outer, n_inner, s);
+    SP_TRY(K128, V128) SP_TRY(K64b, V64) SP_TRY(K64, V64s) SP_TRY(K96, V96) SP_TRY(K256, V256)
+#undef SP_TRY
+    return hipErrorNotSupported;
 }
 
 // In-place round trip of every head's vectors at n_cells cache cells (see

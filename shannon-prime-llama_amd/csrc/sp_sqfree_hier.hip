@@ -297,6 +297,38 @@ hipError_t sp_launch_sqfree_encode(const SpPlan &P, const SpSqGeo &G, const void
     return hipGetLastError();
 }
 
+// K and V of one call: in one launch where the lane kernels take the pair, else one
+// after the other (two sides that share destination bytes keep their order).
+hipError_t sp_launch_sqfree_encode_kv(const SpPlan &KP, const SpPlan &VP, const SpSqGeo &GK, const SpSqGeo &GV,
+                                      const void *src_k, const void *src_v, int dtype, long long so, long long si,
+                                      unsigned char *dst_k, unsigned char *dst_v, long long dout_k, long long dout_v,
+                                      int n_outer, int n_inner, hipStream_t s) {
+    if (n_outer <= 0 || n_inner <= 0) return hipSuccess;
+    if (!getenv_lane_off_sq()) {
+        const hipError_t e = sp_launch_sqfree_encode_lane_kv(KP, VP, GK, GV, src_k, src_v, dtype, so, si, dst_k, dst_v,
+                                                             dout_k, dout_v, n_outer, n_inner, s);
+        if (e != hipErrorNotSupported) return e;
+    }
+    const hipError_t e = sp_launch_sqfree_encode(KP, GK, src_k, dtype, so, si, dst_k, dout_k, n_outer, n_inner, s);
+    if (e != hipSuccess) return e;
+    return sp_launch_sqfree_encode(VP, GV, src_v, dtype, so, si, dst_v, dout_v, n_outer, n_inner, s);
+}
+
+hipError_t sp_launch_sqfree_decode_kv(const SpPlan &KP, const SpPlan &VP, const SpSqGeo &GK, const SpSqGeo &GV,
+                                      const unsigned char *src_k, const unsigned char *src_v, long long so_k,
+                                      long long so_v, void *dst_k, void *dst_v, int dtype, long long dout,
+                                      long long din, int n_outer, int n_inner, hipStream_t s) {
+    if (n_outer <= 0 || n_inner <= 0) return hipSuccess;
+    if (!getenv_lane_off_sq() && sp_kv_rows_disjoint(dst_k, dst_v, dtype, GK.hd, dout, din, n_outer, n_inner)) {
+        const hipError_t e = sp_launch_sqfree_decode_lane_kv(KP, VP, GK, GV, src_k, src_v, so_k, so_v, dst_k, dst_v,
+                                                             dtype, dout, din, n_outer, n_inner, s);
+        if (e != hipErrorNotSupported) return e;
+    }
+    const hipError_t e = sp_launch_sqfree_decode(KP, GK, src_k, so_k, dst_k, dtype, dout, din, n_outer, n_inner, s);
+    if (e != hipSuccess) return e;
+    return sp_launch_sqfree_decode(VP, GV, src_v, so_v, dst_v, dtype, dout, din, n_outer, n_inner, s);
+}
+
 hipError_t sp_launch_sqfree_decode(const SpPlan &P, const SpSqGeo &G, const unsigned char *src,
                                    long long so, void *dst, int dtype, long long dout,
                                    long long din, int n_outer, int n_inner, hipStream_t s, const int *cells) {
@@ -388,7 +420,9 @@ hipError_t sp_launch_hier_decode_kv(const SpPlan &P, const SpHierGeo &G, const u
                                     long long dout, long long din, int n_outer, int n_inner, hipStream_t s) {
     if (n_outer <= 0 || n_inner <= 0) return hipSuccess;
     if (!sq_fits(P, G.pad, G.bytes)) return hipErrorInvalidValue;
-    if (!getenv_lane_off_sq() && sp_hier_split_pays(dtype, 2LL * n_outer * ((n_inner + 63) / 64), 2)) {
+    // two sides that share destination bytes keep their order
+    if (!getenv_lane_off_sq() && sp_hier_split_pays(dtype, 2LL * n_outer * ((n_inner + 63) / 64), 2) &&
+        sp_kv_rows_disjoint(dst_k, dst_v, dtype, G.hd, dout, din, n_outer, n_inner)) {
         const hipError_t e =
             sp_launch_hier_decode_split(P, G, src_k, so, dst_k, dtype, dout, din, n_outer, n_inner, s, src_v, dst_v);
         if (e != hipErrorNotSupported) return e;

@@ -17,23 +17,21 @@
 namespace {
 
 template <int DT, int HD, int PAD, int SK, int RBITS, bool SPIN, class SL>
-__global__ void __launch_bounds__(64)
-k_sqfree_encode_lane(const void *__restrict__ src, long long so, long long si, unsigned char *__restrict__ dst,
-                     long long dout, int n_inner, int tiles_per_outer, int n_tiles, const XfConst K) {
+__device__ __forceinline__ void sq_enc_tiles(const void *src, long long so, long long si, unsigned char *dst,
+                                             long long dout, const TileMap &M, int t, int step, int n_tiles,
+                                             const XfConst &K, unsigned char *rows) {
     using G = SqRec<PAD, SK, RBITS, SPIN, SL>;
     constexpr int RB = row_bytes<DT>(HD), RP = RB + 16, CPR = RB / 16, NR = PAD - SK, DWR = G::dwords;
     constexpr auto &KN = kKnight<PAD, SK>;
     static_assert(SL::hd == SK, "skeleton layout must cover the skeleton");
-    __shared__ __attribute__((aligned(16))) unsigned char rows[64 * RP];  // input rows, then the record stage
-    const int lane = threadIdx.x;
-    const TileMap M{tiles_per_outer, n_inner};
+    const int lane = threadIdx.x;  // rows: the input rows, then the record stage
     // the next tile's rows are in flight while this one computes
     u32x4 pre[CPR];
-    if (blockIdx.x < n_tiles) tile_rows_load<DT, HD>(src, so, si, M, blockIdx.x, lane, pre);
-    for (int t = blockIdx.x; t < n_tiles; t += gridDim.x) {
+    if (t < n_tiles) tile_rows_load<DT, HD>(src, so, si, M, t, lane, pre);
+    for (; t < n_tiles; t += step) {
         uint4 in[CPR];
         tile_rows_put<DT, HD>(pre, lane, rows, in);
-        if (t + (int)gridDim.x < n_tiles) tile_rows_load<DT, HD>(src, so, si, M, t + gridDim.x, lane, pre);
+        if (t + step < n_tiles) tile_rows_load<DT, HD>(src, so, si, M, t + step, lane, pre);
         float c[PAD];
         float mx = 0.0f;
 #pragma unroll
@@ -108,23 +106,50 @@ k_sqfree_encode_lane(const void *__restrict__ src, long long so, long long si, u
 
 template <int DT, int HD, int PAD, int SK, int RBITS, bool SPIN, class SL>
 __global__ void __launch_bounds__(64)
-k_sqfree_decode_lane(const unsigned char *__restrict__ src, long long so, void *__restrict__ dst, long long dout,
-                     long long din, int n_inner, int tiles_per_outer, int n_tiles, const XfConst K) {
+k_sqfree_encode_lane(const void *__restrict__ src, long long so, long long si, unsigned char *__restrict__ dst,
+                     long long dout, int n_inner, int tiles_per_outer, int n_tiles, const XfConst K) {
+    __shared__ __attribute__((aligned(16))) unsigned char rows[64 * (row_bytes<DT>(HD) + 16)];
+    sq_enc_tiles<DT, HD, PAD, SK, RBITS, SPIN, SL>(src, so, si, dst, dout, TileMap{tiles_per_outer, n_inner}, blockIdx.x,
+                                                   gridDim.x, n_tiles, K, rows);
+}
+
+// K and V of one call in one launch: the first half of the grid walks K's tiles,
+// the second half V's (the same tile counts and row strides). Sides of one layout
+// share one body.
+template <int DT, int HD, int PAD, int SK, int RBITS, bool SPIN, class LK, class LV>
+__global__ void __launch_bounds__(64)
+k_sqfree_encode_lane_kv(const void *__restrict__ src_k, const void *__restrict__ src_v, long long so, long long si,
+                        unsigned char *__restrict__ dst_k, unsigned char *__restrict__ dst_v, long long dout_k,
+                        long long dout_v, int n_inner, int tiles_per_outer, int n_tiles, const XfConst K) {
+    __shared__ __attribute__((aligned(16))) unsigned char rows[64 * (row_bytes<DT>(HD) + 16)];
+    const int nb = gridDim.x / 2, b = blockIdx.x;
+    const bool v = b >= nb;
+    const TileMap M{tiles_per_outer, n_inner};
+    if constexpr (std::is_same_v<LK, LV>)
+        sq_enc_tiles<DT, HD, PAD, SK, RBITS, SPIN, LK>(v ? src_v : src_k, so, si, v ? dst_v : dst_k, v ? dout_v : dout_k,
+                                                       M, v ? b - nb : b, nb, n_tiles, K, rows);
+    else if (v)
+        sq_enc_tiles<DT, HD, PAD, SK, RBITS, SPIN, LV>(src_v, so, si, dst_v, dout_v, M, b - nb, nb, n_tiles, K, rows);
+    else
+        sq_enc_tiles<DT, HD, PAD, SK, RBITS, SPIN, LK>(src_k, so, si, dst_k, dout_k, M, b, nb, n_tiles, K, rows);
+}
+
+template <int DT, int HD, int PAD, int SK, int RBITS, bool SPIN, class SL>
+__device__ __forceinline__ void sq_dec_tiles(const unsigned char *src, long long so, void *dst, long long dout,
+                                             long long din, const TileMap &M, int t, int step, int n_tiles,
+                                             const XfConst &K, unsigned char *stage) {
     using G = SqRec<PAD, SK, RBITS, SPIN, SL>;
     constexpr int RP = row_bytes<DT>(HD) + 16, NR = PAD - SK, DWR = G::dwords;
     constexpr auto &KN = kKnight<PAD, SK>;
     static_assert(RecTile<G>::NCK * 1024 + 16 <= 64 * RP, "record tile must fit in the row stage");
-    __shared__ __attribute__((aligned(16))) unsigned char stage[64 * RP];
-    const int lane = threadIdx.x, Gs = gridDim.x;
-    const TileMap M{tiles_per_outer, n_inner};
+    const int lane = threadIdx.x;
     RecTile<G> R;
-    int t = blockIdx.x;
     if (t >= n_tiles) return;
     rec_tile_load<G>(R, src, so, M, t, n_tiles, lane);
-    for (; t < n_tiles; t += Gs) {
+    for (; t < n_tiles; t += step) {
         rec_tile_stage<G>(R, stage, M, t, lane);
         __syncthreads();
-        rec_tile_load<G>(R, src, so, M, t + Gs, n_tiles, lane);
+        rec_tile_load<G>(R, src, so, M, t + step, n_tiles, lane);
         uint32_t rec[DWR];
         rec_from_lds<G>(rec, stage, lane);
         float sk[SK];
@@ -151,6 +176,34 @@ k_sqfree_decode_lane(const unsigned char *__restrict__ src, long long so, void *
         vil_stages<PAD, 0, 1>(c, K);
         tile_rows_out<DT, HD>(c, stage, dst, dout, din, M, t, lane);
     }
+}
+
+template <int DT, int HD, int PAD, int SK, int RBITS, bool SPIN, class SL>
+__global__ void __launch_bounds__(64)
+k_sqfree_decode_lane(const unsigned char *__restrict__ src, long long so, void *__restrict__ dst, long long dout,
+                     long long din, int n_inner, int tiles_per_outer, int n_tiles, const XfConst K) {
+    __shared__ __attribute__((aligned(16))) unsigned char stage[64 * (row_bytes<DT>(HD) + 16)];
+    sq_dec_tiles<DT, HD, PAD, SK, RBITS, SPIN, SL>(src, so, dst, dout, din, TileMap{tiles_per_outer, n_inner},
+                                                   blockIdx.x, gridDim.x, n_tiles, K, stage);
+}
+
+template <int DT, int HD, int PAD, int SK, int RBITS, bool SPIN, class LK, class LV>
+__global__ void __launch_bounds__(64)
+k_sqfree_decode_lane_kv(const unsigned char *__restrict__ src_k, const unsigned char *__restrict__ src_v,
+                        long long so_k, long long so_v, void *__restrict__ dst_k, void *__restrict__ dst_v,
+                        long long dout, long long din, int n_inner, int tiles_per_outer, int n_tiles,
+                        const XfConst K) {
+    __shared__ __attribute__((aligned(16))) unsigned char stage[64 * (row_bytes<DT>(HD) + 16)];
+    const int nb = gridDim.x / 2, b = blockIdx.x;
+    const bool v = b >= nb;
+    const TileMap M{tiles_per_outer, n_inner};
+    if constexpr (std::is_same_v<LK, LV>)
+        sq_dec_tiles<DT, HD, PAD, SK, RBITS, SPIN, LK>(v ? src_v : src_k, v ? so_v : so_k, v ? dst_v : dst_k, dout, din, M,
+                                                       v ? b - nb : b, nb, n_tiles, K, stage);
+    else if (v)
+        sq_dec_tiles<DT, HD, PAD, SK, RBITS, SPIN, LV>(src_v, so_v, dst_v, dout, din, M, b - nb, nb, n_tiles, K, stage);
+    else
+        sq_dec_tiles<DT, HD, PAD, SK, RBITS, SPIN, LK>(src_k, so_k, dst_k, dout, din, M, b, nb, n_tiles, K, stage);
 }
 
 // Listed positions (the dual cache's System 2 rows): lane j of tile t decodes the
@@ -259,6 +312,43 @@ hipError_t sq_dec_cells_launch(const SpPlan &P, const unsigned char *src, long l
     return hipGetLastError();
 }
 
+// Both sides in one launch: a tile keeps its wave for ~17 us (encode) or ~13 us
+// (decode) whatever the call's size, so two launches take twice that until the chip is
+// full, and past it the merged grid has one partial last round instead of two.
+// Measured at sk 115, 8 heads, fp16, merged / one after the other, us: encode 18.5 / 35.8
+// at 1 tile a side, 20.9 / 37.3 at 512, 68.1 / 72.8 at 2048, 129.5 / 137.9 at 4096;
+// decode 13.9 / 26.3, 16.3 / 27.7, 41.3 / 45.8.
+template <int DT, int SK, class LK, class LV>
+hipError_t sq_enc_kv_launch(const SpPlan &P, const void *src_k, const void *src_v, long long so, long long si,
+                            unsigned char *dst_k, unsigned char *dst_v, long long dout_k, long long dout_v,
+                            int n_outer, int n_inner, hipStream_t s) {
+    const int tpo = (n_inner + 63) / 64;
+    const long long n_tiles = (long long)n_outer * tpo;
+    constexpr long long esz = DT == SP_DT_F16 ? 2 : 4;
+    if (n_tiles > 0x7fffffffLL || si < 128 || 64 * si * esz + 128 * esz > 0x7fffffffLL) return hipErrorNotSupported;
+    const dim3 grid(2 * (unsigned)std::min<long long>(n_tiles, std::max(1, resident_blocks(1) / 2))), block(64);
+    hipLaunchKernelGGL((k_sqfree_encode_lane_kv<DT, 128, 154, SK, 3, true, LK, LV>), grid, block, 0, s, src_k, src_v, so,
+                       si, dst_k, dst_v, dout_k, dout_v, n_inner, tpo, (int)n_tiles, xf_const(P));
+    return hipGetLastError();
+}
+
+template <int DT, int SK, class LK, class LV>
+hipError_t sq_dec_kv_launch(const SpPlan &P, const unsigned char *src_k, const unsigned char *src_v, long long so_k,
+                            long long so_v, void *dst_k, void *dst_v, long long dout, long long din, int n_outer,
+                            int n_inner, hipStream_t s) {
+    const int tpo = (n_inner + 63) / 64;
+    const long long n_tiles = (long long)n_outer * tpo;
+    constexpr long long esz = DT == SP_DT_F16 ? 2 : 4;
+    if (n_tiles > 0x7fffffffLL || din < 128 || 64 * din * esz + 128 * esz > 0x7fffffffLL) return hipErrorNotSupported;
+    // fp16 calls past two rounds keep the two launches: V's single band runs faster on the
+    // grid that is not resident (2560 tiles a side: 57.9 us, merged 61.4; fp32 94.6, merged 73.1)
+    if (DT == SP_DT_F16 && n_tiles > resident_blocks(2)) return hipErrorNotSupported;
+    const dim3 grid(2 * (unsigned)std::min<long long>(n_tiles, std::max(1, resident_blocks(2) / 2))), block(64);
+    hipLaunchKernelGGL((k_sqfree_decode_lane_kv<DT, 128, 154, SK, 3, true, LK, LV>), grid, block, 0, s, src_k, src_v,
+                       so_k, so_v, dst_k, dst_v, dout, din, n_inner, tpo, (int)n_tiles, xf_const(P));
+    return hipGetLastError();
+}
+
 }  // namespace
 
 // Listed positions (see k_sqfree_decode_lane_cells); hipErrorNotSupported
@@ -321,5 +411,45 @@ hipError_t sp_launch_sqfree_decode_lane(const SpPlan &P, const SpSqGeo &G, const
     if (sq_geometry_matches<115, SkelL115V3>(P, G))
         return dtype == SP_DT_F16 ? sq_dec_launch<SP_DT_F16, 115, SkelL115V3>(P, src, so, dst, dout, din, n_outer, n_inner, s)
                                   : sq_dec_launch<SP_DT_F32, 115, SkelL115V3>(P, src, so, dst, dout, din, n_outer, n_inner, s);
+    return hipErrorNotSupported;
+}
+
+// K and V in one launch; hipErrorNotSupported (nothing launched) when the pair of
+// geometries or the alignment has no lane specialization.
+hipError_t sp_launch_sqfree_encode_lane_kv(const SpPlan &KP, const SpPlan &VP, const SpSqGeo &GK, const SpSqGeo &GV,
+                                           const void *src_k, const void *src_v, int dtype, long long so, long long si,
+                                           unsigned char *dst_k, unsigned char *dst_v, long long dout_k,
+                                           long long dout_v, int n_outer, int n_inner, hipStream_t s) {
+    const int esz = dtype == SP_DT_F16 ? 2 : 4;
+    if (((uintptr_t)src_k % 16) || ((uintptr_t)src_v % 16) || ((so * esz) % 16) || ((si * esz) % 16) ||
+        ((uintptr_t)dst_k % 2) || ((uintptr_t)dst_v % 2) || (dout_k % 2) || (dout_v % 2))
+        return hipErrorNotSupported;
+#define SP_TRY(SK, LK, LV)                                                                                            \
+    if (sq_geometry_matches<SK, LK>(KP, GK) && sq_geometry_matches<SK, LV>(VP, GV))                                   \
+        return dtype == SP_DT_F16 ? sq_enc_kv_launch<SP_DT_F16, SK, LK, LV>(KP, src_k, src_v, so, si, dst_k, dst_v,   \
+                                                                            dout_k, dout_v, n_outer, n_inner, s)      \
+                                  : sq_enc_kv_launch<SP_DT_F32, SK, LK, LV>(KP, src_k, src_v, so, si, dst_k, dst_v,   \
+                                                                            dout_k, dout_v, n_outer, n_inner, s);
+    SP_TRY(77, SkelL77, SkelL77) SP_TRY(115, SkelL115, SkelL115) SP_TRY(115, SkelL115, SkelL115V3)
+#undef SP_TRY
+    return hipErrorNotSupported;
+}
+
+hipError_t sp_launch_sqfree_decode_lane_kv(const SpPlan &KP, const SpPlan &VP, const SpSqGeo &GK, const SpSqGeo &GV,
+                                           const unsigned char *src_k, const unsigned char *src_v, long long so_k,
+                                           long long so_v, void *dst_k, void *dst_v, int dtype, long long dout,
+                                           long long din, int n_outer, int n_inner, hipStream_t s) {
+    const int esz = dtype == SP_DT_F16 ? 2 : 4;
+    if (((uintptr_t)dst_k % 16) || ((uintptr_t)dst_v % 16) || ((dout * esz) % 16) || ((din * esz) % 16) ||
+        ((uintptr_t)src_k % 2) || ((uintptr_t)src_v % 2) || (so_k % 2) || (so_v % 2))
+        return hipErrorNotSupported;
+#define SP_TRY(SK, LK, LV)                                                                                            \
+    if (sq_geometry_matches<SK, LK>(KP, GK) && sq_geometry_matches<SK, LV>(VP, GV))                                   \
+        return dtype == SP_DT_F16 ? sq_dec_kv_launch<SP_DT_F16, SK, LK, LV>(KP, src_k, src_v, so_k, so_v, dst_k,      \
+                                                                            dst_v, dout, din, n_outer, n_inner, s)    \
+                                  : sq_dec_kv_launch<SP_DT_F32, SK, LK, LV>(KP, src_k, src_v, so_k, so_v, dst_k,      \
+                                                                            dst_v, dout, din, n_outer, n_inner, s);
+    SP_TRY(77, SkelL77, SkelL77) SP_TRY(115, SkelL115, SkelL115) SP_TRY(115, SkelL115, SkelL115V3)
+#undef SP_TRY
     return hipErrorNotSupported;
 }

@@ -114,3 +114,40 @@ def test_sqfree_layer(v_bits, n, start):
 
     _check(cc, S.lib().sp_hip_sqfree_write_layer, read, [comp(0), comp(1)], [dec(0), dec(1)],
            [cc.c.bytes_per_pos_k, cc.c.bytes_per_pos_v], hd, n, start, False)
+
+
+@pytest.mark.parametrize("kind", ["ship", "sqfree", "hier"])
+def test_sides_read_into_one_buffer(kind):
+    """Both sides of a read in one buffer: interleaved rows (K and V of a token side by side)
+    give what separate buffers give; the same rows for both end with V's, as two reads would."""
+    H, n, start = 2, 150, 1
+    hd = 256 if kind == "hier" else 128
+    ms = start + n + 3
+    say(f"lane cells one buffer {kind}")
+    stream = torch.cuda.current_stream().cuda_stream
+    if kind == "ship":
+        cc = S.ShipCache(S.config(hd, 1, H), ms, stream=stream)
+        write, rd = S.lib().sp_hip_write_layer, S.lib().sp_hip_read_layer
+        tail = (-1,)
+    elif kind == "sqfree":
+        b = [5, 4, 4, 4, 5]
+        cc = S.SqfreeCache(S.config(hd, 1, H, k_bits=b, v_bits=b), ms, rbits=3, spinor=True, sk_k=77, stream=stream)
+        write, rd, tail = S.lib().sp_hip_sqfree_write_layer, S.lib().sp_hip_sqfree_read_layer, ()
+    else:
+        sk, tg = O.hier_geometry(330)
+        cc = S.HierCache(S.config(hd, 1, H), 330, sk, tg, S.band_config(len(sk), [5, 5]), 2, ms, H, stream=stream)
+        cc.upload_W(W.hier_W(H, len(tg), len(sk), seed=4))
+        write, rd, tail = S.lib().sp_hip_hier_write_layer, S.lib().sp_hip_hier_read_layer, ()
+    w = H * hd
+    t = [dev(x.view(np.uint16).transpose(1, 0, 2).reshape(n, w)) for x in W.cfg1_kv(n_heads=H, n_pos=n, hd=hd, seed=3)]
+    S.check(write(cc.ref, 0, start, n, p(t[0]), p(t[1]), w, S.DTYPE_F16))
+    ref = [torch.zeros((n, w), dtype=torch.int16, device="cuda") for _ in range(2)]
+    S.check(rd(cc.ref, 0, start, n, p(ref[0]), p(ref[1]), w, S.DTYPE_F16, *tail))
+    mixed = torch.zeros((n, 2, w), dtype=torch.int16, device="cuda")
+    S.check(rd(cc.ref, 0, start, n, p(mixed), p(mixed[0, 1]), 2 * w, S.DTYPE_F16, *tail))
+    one = torch.zeros((n, w), dtype=torch.int16, device="cuda")
+    S.check(rd(cc.ref, 0, start, n, p(one), p(one), w, S.DTYPE_F16, *tail))
+    torch.cuda.synchronize()
+    assert torch.equal(mixed[:, 0], ref[0]) and torch.equal(mixed[:, 1], ref[1])
+    assert torch.equal(one, ref[1]) and not torch.equal(ref[0], ref[1])
+    cc.free()
