@@ -21,8 +21,10 @@
 // decodes it (compile-time Knight CSR and record fields), the scores as dot products
 // with the prepared queries, an online softmax across the run's tiles, and the
 // weighted coefficient sums through LDS (the wave's coefficients transposed so that
-// each lane sums one coefficient over the tile's 64 positions).
+// each lane sums one coefficient over the tile's 64 positions); both products on the
+// matrix cores in fp32.
 #include <cstdlib>
+#include <utility>
 
 #include "sp_sqfree_lane.h"
 
@@ -58,20 +60,77 @@ __device__ __forceinline__ void sq_coefficients(const uint32_t (&rec)[DW], float
 // wave reductions on DPP and the row swaps (every lane active at each call)
 __device__ __forceinline__ float wave_max(float v) { return sp_wave_max_dpp(v); }
 __device__ __forceinline__ float wave_add(float v) { return sp_wave_sum_dpp(v); }
+// a value that every lane holds, in a scalar register
+__device__ __forceinline__ float wave_uniform(float v) {
+    return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(v)));
+}
 
-// The score factors of one query head in chunks of at most 16: the skeleton part
-// (SK factors) then the residual part (PAD - SK), a chunk never spanning both.
-template <int SK, int PAD>
-struct QChunks {
-    static constexpr int NS = (SK + 15) / 16, NR = (PAD - SK + 15) / 16, N = NS + NR;
-    // coefficient index of chunk k's first factor, and the chunk's factor count
-    static constexpr int first(int k) { return k < NS ? 16 * k : SK + 16 * (k - NS); }
-    static constexpr int size(int k) {
-        return k < NS ? (SK - 16 * k < 16 ? SK - 16 * k : 16) : (PAD - SK - 16 * (k - NS) < 16 ? PAD - SK - 16 * (k - NS) : 16);
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+// Sixteen 4x4x1 fp32 products in one matrix instruction, each of the sixteen 4-lane
+// blocks taking its A rows from block AB of its group of 2^CB blocks: with CB = 4,
+// c[i](lane) += a(lane 4*AB + i) * b(lane) for i < 4. An fp32 fused multiply-add of
+// four query heads' factors with a value per lane, at twice the vector unit's rate
+// and without the factors in scalar registers.
+template <int CB, int AB>
+__device__ __forceinline__ f32x4 fma_heads(float a, float b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_4x4x1f32(a, b, c, CB, AB, 0);
+}
+
+constexpr int NQ = (PAD + 15) / 16;  // registers of one head group's factors, 16 coefficients each
+
+// scores: s[g][C % 3][i](position) += q~[4g + i][C] * e[C](position), every C of the pack
+template <int NG, int C>
+__device__ __forceinline__ void score_step(const float (&q)[NG][NQ], const float (&e)[PAD], f32x4 (&s)[NG][3]) {
+#pragma unroll
+    for (int g = 0; g < NG; g++) s[g][C % 3] = fma_heads<4, C % 16>(q[g][C / 16], e[C], s[g][C % 3]);
+}
+template <int NG, int... C>
+__device__ __forceinline__ void score_all(const float (&q)[NG][NQ], const float (&e)[PAD], f32x4 (&s)[NG][3],
+                                          std::integer_sequence<int, C...>) {
+    (score_step<NG, C>(q, e, s), ...);
+}
+
+// weighted sums: acc[g][i](coefficient) += p[4g + i][position] * E[coefficient][position]
+// for the four positions 4*K .. 4*K + 3 of the row ei (PER positions per weight register)
+template <int NG, int PER, int CB, int K, int NP>
+__device__ __forceinline__ void sum_step(const float (&pw)[NG][NP], const f32x4 &ei, f32x4 (&acc)[NG]) {
+#pragma unroll
+    for (int g = 0; g < NG; g++) {
+        acc[g] = fma_heads<CB, (4 * K + 0) % PER>(pw[g][4 * K / PER], ei[0], acc[g]);
+        acc[g] = fma_heads<CB, (4 * K + 1) % PER>(pw[g][4 * K / PER], ei[1], acc[g]);
+        acc[g] = fma_heads<CB, (4 * K + 2) % PER>(pw[g][4 * K / PER], ei[2], acc[g]);
+        acc[g] = fma_heads<CB, (4 * K + 3) % PER>(pw[g][4 * K / PER], ei[3], acc[g]);
     }
-};
+}
+// all of a row's positions, sixteen at a time: the next sixteen are read while these
+// multiply, and no more (the barriers keep the rest of the reads behind)
+template <int NG, int PER, int CB, int N16, int J, int NP>
+__device__ __forceinline__ void sum_16(const float (&pw)[NG][NP], const float *row, const f32x4 (&ei)[4],
+                                       f32x4 (&acc)[NG]) {
+    f32x4 en[4];
+    if constexpr (J + 1 < N16) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) en[k] = *reinterpret_cast<const f32x4 *>(row + 16 * (J + 1) + 4 * k);
+    }
+    sum_step<NG, PER, CB, 4 * J + 0>(pw, ei[0], acc);
+    sum_step<NG, PER, CB, 4 * J + 1>(pw, ei[1], acc);
+    sum_step<NG, PER, CB, 4 * J + 2>(pw, ei[2], acc);
+    sum_step<NG, PER, CB, 4 * J + 3>(pw, ei[3], acc);
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (J + 1 < N16) sum_16<NG, PER, CB, N16, J + 1>(pw, row, en, acc);
+}
+template <int NG, int PER, int CB, int N16, int NP>
+__device__ __forceinline__ void sum_all(const float (&pw)[NG][NP], const float *row, f32x4 (&acc)[NG]) {
+    f32x4 ei[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) ei[k] = *reinterpret_cast<const f32x4 *>(row + 4 * k);
+    sum_16<NG, PER, CB, N16, 0>(pw, row, ei, acc);
+}
 
-constexpr int EP = 65;  // LDS row pitch (floats) of the transposed coefficient chunk
+// LDS row pitch (floats) of the transposed coefficient chunk: 16-byte rows, eight lanes'
+// 16-byte pieces on distinct banks
+constexpr int EP = 68;
 
 // Scores, online softmax and the V records' weighted coefficient sums. Block
 // (kvh, run) takes tiles run, run + n_runs, ... of KV head kvh (64 positions each).
@@ -80,6 +139,21 @@ constexpr int EP = 65;  // LDS row pitch (floats) of the transposed coefficient 
 // residual part's offset. Partial per (query head, run) at part + ((h0 + h) * n_runs
 // + run) * pp: [m, l, 0, 0, sum p c~ (PAD coefficients, skeleton then residuals)].
 // OUT = false: scores only.
+//
+// Both contractions run on the matrix cores in fp32 (fma_heads), four query heads at a
+// time: the scores with the prepared queries in registers (lane 4b + i of register j:
+// head i of the group, coefficient 16j + b) against the lane's own coefficients, in three
+// chains of sums; the weighted sums with the tile's weights (lane 4b + i of register j:
+// head i, position 16j + b) against the transposed chunk (lane = coefficient, four
+// positions per 16-byte LDS read).
+//
+// Bound by the decode of the two records (2400 vector instructions a tile beside 628
+// matrix instructions) and by latency at two waves per SIMD, which the 154 coefficients a
+// lane holds allow at most. Four sequences of 16384 over 4 KV heads and 8 query heads
+// each: 71 us with the products on the vector unit (4900 instructions a tile, queries and
+// weights by scalar loads and LDS broadcasts), 48 us now. Two chains of sums took 45 us and
+// four 50; the mean error against 64-bit results over 126 shapes was 4.6e-7 with two,
+// 3.9e-7 with three, 3.6e-7 with four, and 4.5e-7 before.
 template <int SK, class SLK, class SLV, int GM, bool OUT>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2)))
 k_sqfree_attn_split(const unsigned char *__restrict__ kc0, const unsigned char *__restrict__ vc0, long long k_slot,
@@ -89,8 +163,8 @@ k_sqfree_attn_split(const unsigned char *__restrict__ kc0, const unsigned char *
     using GV = SqRec<PAD, SK, RBITS, true, SLV>;
     constexpr int NCK = RecTile<GK>::NCK > RecTile<GV>::NCK ? RecTile<GK>::NCK : RecTile<GV>::NCK;
     constexpr int C2 = PAD - 128;  // coefficients of the third 64-coefficient chunk
-    constexpr int HG = (GM + 1) / 2;  // heads per lane in the third chunk (two lanes per coefficient)
-    static_assert(C2 > 0 && 2 * C2 <= 64, "three chunks of at most 64 coefficients");
+    constexpr int NG = (GM + 3) / 4;  // groups of four query heads
+    static_assert(C2 > 0 && C2 <= 32, "two whole chunks, and one of at most 32 coefficients");
     // the record stage and the transposed coefficient chunks share their memory: in
     // this one-wave block the stage's last reads (the V records) come before the first
     // chunk's writes, and the next tile's K records are staged after the last chunk's
@@ -98,7 +172,7 @@ k_sqfree_attn_split(const unsigned char *__restrict__ kc0, const unsigned char *
     __shared__ __attribute__((aligned(16))) float E[OUT ? 64 * EP : (NCK * 1024 + 16 + 3) / 4];
     static_assert(NCK * 1024 + 16 <= 64 * EP * 4, "the record stage fits the chunk memory");
     unsigned char *const stage = reinterpret_cast<unsigned char *>(E);
-    __shared__ __attribute__((aligned(16))) float Pw[64 * GM];
+    __shared__ __attribute__((aligned(16))) f32x4 Pw[OUT ? 64 * NG : 1];  // [position][group]
     // block x: head group x (query heads x G .. x G + G - 1) of KV head x / hs
     const int hb = blockIdx.x, kvh = hb / hs, run = blockIdx.y, lane = threadIdx.x;
     // sequence blockIdx.z: its positions, prepared queries, score rows and partials
@@ -115,19 +189,20 @@ k_sqfree_attn_split(const unsigned char *__restrict__ kc0, const unsigned char *
     const TileMap M{tpo, n_kv};
     const float *__restrict__ pq = prep + (long long)h0 * ps;
 
+    const int lb = lane / 4, li = lane % 4;
+    const f32x4 z4 = {0.0f, 0.0f, 0.0f, 0.0f};
     float m_run[GM], l_run[GM];
-    float acc0[GM], acc1[GM], acc2[HG];
+    f32x4 acc0[NG], acc1[NG], acc2[NG];
 #pragma unroll
     for (int h = 0; h < GM; h++) {
         m_run[h] = -INFINITY;
         l_run[h] = 0.0f;
-        acc0[h] = acc1[h] = 0.0f;
     }
 #pragma unroll
-    for (int h = 0; h < HG; h++) acc2[h] = 0.0f;
-    // third chunk: coefficient 128 + c2i for heads hh * HG .. hh * HG + HG - 1
-    const int c2i = lane % C2, hh = lane / C2;
-    const bool c2_on = hh < (GM > 1 ? 2 : 1);
+    for (int g = 0; g < NG; g++) acc0[g] = acc1[g] = acc2[g] = z4;
+    // third chunk: lane = coefficient 128 + c2i, positions 32 * half .. 32 * half + 31
+    // (the two halves are added at the end)
+    const int half = lane / 32, c2i = lane % 32 < C2 ? lane % 32 : C2 - 1;
 
     // a tile's K and V records load at the tile's start (holding the next tile's K records
     // through a tile took the registers that keep the full instances from spilling at two
@@ -138,6 +213,25 @@ k_sqfree_attn_split(const unsigned char *__restrict__ kc0, const unsigned char *
         rec_tile_load<GK>(Rk, kc, k_slot, M, t, n_tiles, lane);
         RecTile<GV> Rv;
         if (OUT) rec_tile_load<GV>(Rv, vc, v_slot, M, t, n_tiles, lane);
+        // the head groups' factors, again for each tile (cache hits beside the records' loads):
+        // held across the V half they cost the registers that keep it from spilling
+        float q[NG][NQ];
+        int zero = 0;
+        __asm__ volatile("" : "+v"(zero));  // no hoisting out of the tile loop
+#pragma unroll
+        for (int g = 0; g < NG; g++) {
+            // heads past the group's and coefficients past the pad repeat the last: their
+            // products are never read
+            const int h = 4 * g + li < G ? 4 * g + li : G - 1, o = h * ps + lb + zero;
+#pragma unroll
+            for (int j = 0; j < NQ; j++) {
+                const int k = 16 * j;  // coefficients k + lb
+                if (k + 16 <= SK) q[g][j] = pq[o + k];
+                else if (k >= SK && k + 16 <= PAD) q[g][j] = pq[o + k + (qo - SK)];
+                else if (k < SK) q[g][j] = pq[o + k + (k + lb < SK ? 0 : qo - SK)];
+                else q[g][j] = pq[o + (k + lb < PAD ? k : PAD - 1 - lb) + (qo - SK)];
+            }
+        }
         __syncthreads();  // the previous tile is done with the stage
         rec_tile_stage<GK>(Rk, stage, M, t, lane);
         __syncthreads();
@@ -147,66 +241,40 @@ k_sqfree_attn_split(const unsigned char *__restrict__ kc0, const unsigned char *
         sq_coefficients<SK, SLK>(rk, e);
         const int pos = c * 64 + lane;
         const bool live = pos < n_kv;
+        f32x4 s3[NG][3];
+#pragma unroll
+        for (int g = 0; g < NG; g++) s3[g][0] = s3[g][1] = s3[g][2] = z4;
+        score_all<NG>(q, e, s3, std::make_integer_sequence<int, PAD>{});
         float s[GM];
 #pragma unroll
         for (int h = 0; h < GM; h++) {
             s[h] = -INFINITY;
-            if (h < G) {
-                // q~ . e: the head's factors are wave-uniform and arrive by scalar loads,
-                // 16 at a time. In the full instances chunk k + 1 is loaded after the first
-                // product of chunk k (a scalar-load wait covers every scalar load in flight,
-                // so the next chunk cannot go out before the wait for the current one):
-                // 2% faster there; the scores-only instances measured 4% slower with it and
-                // keep the compiler's placement.
-                const float *__restrict__ qh = pq + h * ps;
-                using QC = QChunks<SK, PAD>;
-                float qa[16], qb[16];
-#pragma unroll
-                for (int i = 0; i < QC::size(0); i++) qa[i] = qh[i];
-                float a0 = 0.0f, a1 = 0.0f;
-#pragma unroll
-                for (int k = 0; k < QC::N; k++) {
-                    float(&q)[16] = (k & 1) ? qb : qa;
-                    float(&qn)[16] = (k & 1) ? qa : qb;
-                    const int e0 = QC::first(k);
-                    a0 = fmaf(q[0], e[e0], a0);
-                    if (k + 1 < QC::N) {
-                        const float *__restrict__ qs = qh + (k + 1 < QC::NS ? 16 * (k + 1) : qo + 16 * (k + 1 - QC::NS));
-                        if constexpr (OUT) __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                        for (int i = 0; i < QC::size(k + 1); i++) qn[i] = qs[i];
-                        if constexpr (OUT) __builtin_amdgcn_sched_barrier(0);
-                    }
-#pragma unroll
-                    for (int i = 1; i < QC::size(k); i++) {
-                        if (i & 1) a1 = fmaf(q[i], e[e0 + i], a1);
-                        else a0 = fmaf(q[i], e[e0 + i], a0);
-                    }
-                }
-                const float v = a0 + a1;
-                if (live) {
-                    s[h] = v;
-                    if (scores) scores[(long long)(h0 + h) * s_stride + pos] = v;
-                }
+            if (h < G && live) {
+                const f32x4(&v)[3] = s3[h / 4];
+                s[h] = (v[0][h % 4] + v[1][h % 4]) + v[2][h % 4];
+                if (scores) scores[(long long)(h0 + h) * s_stride + pos] = s[h];
             }
         }
         if (!OUT) continue;
         // ---- online softmax over the tile (wave-wide per head) ----
         float alpha[GM];
+        f32x4 pr[NG];
+#pragma unroll
+        for (int g = 0; g < NG; g++) pr[g] = z4;
 #pragma unroll
         for (int h = 0; h < GM; h++) {
             alpha[h] = 1.0f;
             if (h < G) {
                 const float mn = fmaxf(m_run[h], wave_max(s[h]));
-                alpha[h] = __expf(m_run[h] - mn);
-                const float pr = live ? __expf(s[h] - mn) : 0.0f;
-                l_run[h] = fmaf(l_run[h], alpha[h], wave_add(pr));
-                m_run[h] = mn;
-                Pw[lane * GM + h] = pr;
-            } else {
-                Pw[lane * GM + h] = 0.0f;
+                alpha[h] = wave_uniform(__expf(m_run[h] - mn));
+                const float p = live ? __expf(s[h] - mn) : 0.0f;
+                l_run[h] = wave_uniform(fmaf(l_run[h], alpha[h], wave_add(p)));
+                m_run[h] = wave_uniform(mn);
+                pr[h / 4][h % 4] = p;
             }
         }
+#pragma unroll
+        for (int g = 0; g < NG; g++) Pw[lane * NG + g] = pr[g];
         // ---- V records of the tile, then their coefficients ----
         __syncthreads();  // every lane has read its K record from the stage
         rec_tile_stage<GV>(Rv, stage, M, t, lane);
@@ -217,19 +285,18 @@ k_sqfree_attn_split(const unsigned char *__restrict__ kc0, const unsigned char *
         sq_coefficients<SK, SLV>(rv, ev);
 #pragma unroll
         for (int h = 0; h < GM; h++) {
-            acc0[h] *= alpha[h];
-            acc1[h] *= alpha[h];
-        }
-#pragma unroll
-        for (int k = 0; k < HG; k++) {
-            float a = 1.0f;
-#pragma unroll
-            for (int h = 0; h < GM; h++)
-                if (h == hh * HG + k) a = alpha[h];
-            acc2[k] *= a;
+            acc0[h / 4][h % 4] *= alpha[h];
+            acc1[h / 4][h % 4] *= alpha[h];
+            acc2[h / 4][h % 4] *= alpha[h];
         }
         // ---- weighted coefficient sums: chunk of 64 coefficients transposed through
         // LDS (row = coefficient, column = position), lane = coefficient ----
+        const float *const pf = reinterpret_cast<const float *>(Pw);
+        float pw[NG][4];  // lane 4b + i, register j: head i, position 16j + b
+#pragma unroll
+        for (int g = 0; g < NG; g++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) pw[g][j] = pf[(16 * j + lb) * (4 * NG) + 4 * g + li];
 #pragma unroll
         for (int ch = 0; ch < 3; ch++) {
             const int i0 = 64 * ch, n_i = ch < 2 ? 64 : C2;
@@ -238,27 +305,17 @@ k_sqfree_attn_split(const unsigned char *__restrict__ kc0, const unsigned char *
                 if (i < n_i) E[i * EP + lane] = ev[i0 + i];
             __syncthreads();
             if (ch == 0) {
-#pragma unroll 4
-                for (int p = 0; p < 64; p++) {
-                    const float ei = E[lane * EP + p];
-#pragma unroll
-                    for (int h = 0; h < GM; h++) acc0[h] = fmaf(Pw[p * GM + h], ei, acc0[h]);
-                }
+                sum_all<NG, 16, 4, 4>(pw, E + lane * EP, acc0);
             } else if (ch == 1) {
-#pragma unroll 4
-                for (int p = 0; p < 64; p++) {
-                    const float ei = E[lane * EP + p];
+                sum_all<NG, 16, 4, 4>(pw, E + lane * EP, acc1);
+            } else {
+                // half h of the wave: head i, position 32h + 8j + b of its eight blocks b
 #pragma unroll
-                    for (int h = 0; h < GM; h++) acc1[h] = fmaf(Pw[p * GM + h], ei, acc1[h]);
-                }
-            } else if (c2_on) {
-                // hh * HG + k < GM for every lane with c2_on (two halves of HG heads)
-#pragma unroll 4
-                for (int p = 0; p < 64; p++) {
-                    const float ei = E[c2i * EP + p];
+                for (int g = 0; g < NG; g++)
 #pragma unroll
-                    for (int k = 0; k < HG; k++) acc2[k] = fmaf(Pw[p * GM + hh * HG + k], ei, acc2[k]);
-                }
+                    for (int j = 0; j < 4; j++)
+                        pw[g][j] = pf[(32 * half + 8 * j + lb % 8) * (4 * NG) + 4 * g + li];
+                sum_all<NG, 8, 3, 2>(pw, E + c2i * EP + 32 * half, acc2);
             }
             __syncthreads();
         }
@@ -267,6 +324,7 @@ k_sqfree_attn_split(const unsigned char *__restrict__ kc0, const unsigned char *
     // ---- the run's partial per query head ----
 #pragma unroll
     for (int h = 0; h < GM; h++) {
+        const float a2 = acc2[h / 4][h % 4] + __shfl_xor(acc2[h / 4][h % 4], 32);
         if (h >= G) continue;
         float *dst = part + ((long long)(h0 + h) * n_runs + run) * pp;
         if (lane == 0) {
@@ -275,15 +333,9 @@ k_sqfree_attn_split(const unsigned char *__restrict__ kc0, const unsigned char *
             dst[2] = 0.0f;
             dst[3] = 0.0f;
         }
-        dst[4 + lane] = acc0[h];
-        dst[4 + 64 + lane] = acc1[h];
-    }
-    if (c2_on) {
-#pragma unroll
-        for (int k = 0; k < HG; k++) {
-            const int h = hh * HG + k;
-            if (h < G) part[((long long)(h0 + h) * n_runs + run) * pp + 4 + 128 + c2i] = acc2[k];
-        }
+        dst[4 + lane] = acc0[h / 4][h % 4];
+        dst[4 + 64 + lane] = acc1[h / 4][h % 4];
+        if (lane < C2) dst[4 + 128 + lane] = a2;
     }
 }
 
