@@ -198,8 +198,10 @@ __device__ __forceinline__ void split_hl(float v, uint32_t &hi, uint32_t &lo) {
     lo = (uint32_t)__builtin_bit_cast(unsigned short, l);
 }
 
-// Power of two p with amax * p in [2^11, 2^12) (1 when amax is 0 or not finite),
-// and its reciprocal (exact).
+// Power of two p with amax * p in [2^11, 2^12) (1 when amax is 0 or not finite), and its
+// reciprocal (exact). An amax below 2^-113 takes the p of 2^-113: p and 1/p, also with the
+// weights' 2^-6 on them, stay normal numbers (an infinite p would make a NaN of every zero),
+// and what it scales still has its fp32 precision down to about 2^-126.
 __device__ __forceinline__ float pow2_norm(float amax, float &inv) {
     if (!(amax > 0.0f) || !(amax < INFINITY)) {
         inv = 1.0f;
@@ -207,6 +209,7 @@ __device__ __forceinline__ float pow2_norm(float amax, float &inv) {
     }
     int e;
     (void)frexpf(amax, &e);  // amax = f * 2^e, f in [0.5, 1)
+    e = max(e, -112);
     inv = ldexpf(1.0f, e - 12);
     return ldexpf(1.0f, 12 - e);
 }
