@@ -198,18 +198,19 @@ __device__ __forceinline__ void split_hl(float v, uint32_t &hi, uint32_t &lo) {
     lo = (uint32_t)__builtin_bit_cast(unsigned short, l);
 }
 
-// Power of two p with amax * p in [2^11, 2^12) (1 when amax is 0 or not finite), and its
-// reciprocal (exact). An amax below 2^-113 takes the p of 2^-113: p and 1/p, also with the
-// weights' 2^-6 on them, stay normal numbers (an infinite p would make a NaN of every zero),
-// and what it scales still has its fp32 precision down to about 2^-126.
+// Power of two p with amax * p in [2^11, 2^12) (1 when amax is not finite), and its
+// reciprocal (exact). An amax below 2^-113, zero too, takes the p of 2^-113: p and 1/p, also
+// with the weights' 2^-6 on them, stay normal numbers (an infinite p would make a NaN of
+// every zero), what it scales still has its fp32 precision down to about 2^-126, and a wave
+// that has seen no weight yet keeps the largest p there is, so the first one sets its own.
 __device__ __forceinline__ float pow2_norm(float amax, float &inv) {
-    if (!(amax > 0.0f) || !(amax < INFINITY)) {
+    if (!(amax < INFINITY)) {
         inv = 1.0f;
         return 1.0f;
     }
     int e;
     (void)frexpf(amax, &e);  // amax = f * 2^e, f in [0.5, 1)
-    e = max(e, -112);
+    e = amax > 0.0f ? max(e, -112) : -112;
     inv = ldexpf(1.0f, e - 12);
     return ldexpf(1.0f, 12 - e);
 }
@@ -756,7 +757,8 @@ k_attn_wave(const SpAttnArgs A, const int *__restrict__ order, float *__restrict
         // first tile's (largest weight in [2^5, 2^6)) and stay while every weight stays within
         // 2^15, so a usual tile needs no reduction across lanes and no rescaling; the lo parts
         // still resolve 2^-35. A head that outgrows them takes the tile's maximum as its m and
-        // rescales its sums. ----
+        // rescales its sums; so does one whose tiles had zero V records only, at its first
+        // weight (f is the largest there is until then). ----
         unsigned short *wt = reinterpret_cast<unsigned short *>(wl);
         float *stt = reinterpret_cast<float *>(wl + LY::R_ST);
         const float sv[4] = {quad_bcast<0>(sv_own), quad_bcast<1>(sv_own), quad_bcast<2>(sv_own), quad_bcast<3>(sv_own)};

@@ -1,6 +1,6 @@
 """The matrix-core decode attention's powers of two (k_attn_wave: the scale of a head's fp16
-weights and of its query) where what they scale is tiny; against the oracle (1e-3 relative,
-elementwise)."""
+weights and of its query) where what they scale is tiny or a wave's first tiles have no values;
+against the oracle (1e-3 relative, elementwise)."""
 import ctypes as C
 import math
 
@@ -15,7 +15,7 @@ import sp_hip as S  # noqa: E402
 from gpu_util import dev, empty_f32, host, p, stream  # noqa: E402
 from test_gpu_attn import rel_close, say  # noqa: E402
 from test_gpu_attn_seqs import _arr  # noqa: E402
-from test_gpu_attn_wave import LAYOUTS  # noqa: E402
+from test_gpu_attn_wave import BRIDGE, LAYOUTS, SHIP  # noqa: E402
 
 
 def _run(hd, bands, H, n_q, score, v_amp, n_seq=1, q_scale=1.0):
@@ -68,3 +68,20 @@ def test_tiny_query(hd, bands):
     """A query of about 1e-36 (2^-120): its normalising power of two is past the fp32 range."""
     say(f"wave attn tiny query hd={hd} bands={bands}")
     _run(hd, bands, 2, 6, np.linspace(-1.0, 1.0, 200), np.ones(200), q_scale=1e-36)
+
+
+# two or more tiles per wave on 256 CUs
+SEVERAL = [(64, BRIDGE, 8, 2, 16, 2100), (64, SHIP, 8, 8, 16, 3090), (96, BRIDGE, 8, 5, 16, 3100),
+           (96, BRIDGE, 32, 1, 12, 1100), (128, SHIP, 8, 4, 16, 3100), (256, SHIP, 8, 2, 16, 1100),
+           (256, SHIP, 4, 6, 16, 2110)]
+
+
+@pytest.mark.parametrize("lower", [10.0, 20.0])
+@pytest.mark.parametrize("hd,bands,H,G,n_seq,n", SEVERAL)
+def test_first_tiles_without_values(hd, bands, H, G, n_seq, n, lower):
+    """Seven tiles of eight have zero V records; the eighth's scores are 10 or 20 lower and its V
+    records small (scales of about 2^-6): all that the output consists of."""
+    say(f"wave attn no values first hd={hd} bands={bands} H={H} G={G} n={n} lower={lower}")
+    eighth = np.arange(n) // 64 % 8 == 7
+    score = np.where(eighth, -lower, -0.5) + np.random.default_rng(n).uniform(-0.5, 0.5, n)
+    _run(hd, bands, H, H * G, score, np.where(eighth, 0.05, 0.0), n_seq)
