@@ -755,10 +755,12 @@ k_attn_wave(const SpAttnArgs A, const int *__restrict__ order, float *__restrict
         // ---- softmax weights, lane (quad qd, head hj) holding positions 4*qd + i; w =
         // p * scale_v * f as fp16 hi / lo rows 2h / 2h + 1 (slot = position). m and f are the
         // first tile's (largest weight in [2^5, 2^6)) and stay while every weight stays within
-        // 2^15, so a usual tile needs no reduction across lanes and no rescaling; the lo parts
-        // still resolve 2^-35. A head that outgrows them takes the tile's maximum as its m and
-        // rescales its sums; so does one whose tiles had zero V records only, at its first
-        // weight (f is the largest there is until then). ----
+        // 2^15 and every p within 2^60, so a usual tile needs no reduction across lanes and no
+        // rescaling; the lo parts still resolve 2^-35. A head that outgrows them takes the
+        // tile's maximum as its m and rescales its sums; so does one whose tiles had zero V
+        // records only, at its first weight (f is the largest there is until then). (p has a
+        // bound of its own for positions whose V record is zero: its weight stays 0, or is
+        // inf * 0, however far its score is above m.) ----
         unsigned short *wt = reinterpret_cast<unsigned short *>(wl);
         float *stt = reinterpret_cast<float *>(wl + LY::R_ST);
         const float sv[4] = {quad_bcast<0>(sv_own), quad_bcast<1>(sv_own), quad_bcast<2>(sv_own), quad_bcast<3>(sv_own)};
@@ -770,14 +772,16 @@ k_attn_wave(const SpAttnArgs A, const int *__restrict__ order, float *__restrict
             for (int i = 0; i < 4; i++) v[st][i] = 4 * qd + i < n_chunk ? sc[st][i] : -INFINITY;  // past the tile's end: no weight
             grown[st] = false;
             if (MULTI) {
-                float wm = 0.0f;
+                float wm = 0.0f, pm = 0.0f;
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
                     pr[st][i] = __expf(v[st][i] - m_run[st]);
                     wx[st][i] = pr[st][i] * sv[i] * f_run[st];
                     wm = fmaxf(wm, wx[st][i]);
+                    pm = fmaxf(pm, pr[st][i]);
                 }
-                grown[st] = 4 * st + hj < G && !(wm <= 32768.0f);
+                // both bounds in one: 2^60 * 2^-45 is 2^15 (and an infinite p passes it)
+                grown[st] = 4 * st + hj < G && !(fmaf(pm, 0x1p-45f, wm) <= 32768.0f);
                 any_grown = any_grown || grown[st];
             }
         }

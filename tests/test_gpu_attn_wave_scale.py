@@ -1,6 +1,7 @@
 """The matrix-core decode attention's powers of two (k_attn_wave: the scale of a head's fp16
-weights and of its query) where what they scale is tiny or a wave's first tiles have no values;
-against the oracle (1e-3 relative, elementwise)."""
+weights and of its query) where what they scale is tiny or a wave's first tiles have no values,
+and its softmax reference where a later best score has no value; against the oracle (1e-3
+relative, elementwise)."""
 import ctypes as C
 import math
 
@@ -85,3 +86,16 @@ def test_first_tiles_without_values(hd, bands, H, G, n_seq, n, lower):
     eighth = np.arange(n) // 64 % 8 == 7
     score = np.where(eighth, -lower, -0.5) + np.random.default_rng(n).uniform(-0.5, 0.5, n)
     _run(hd, bands, H, H * G, score, np.where(eighth, 0.05, 0.0), n_seq)
+
+
+@pytest.mark.parametrize("above", [40.0, 95.0])
+@pytest.mark.parametrize("hd,bands,H,G,n_seq,n", SEVERAL)
+def test_later_best_position_without_values(hd, bands, H, G, n_seq, n, above):
+    """One position of the eighth tile scores 40 or 95 above its wave's first tile (past the range
+    of the fp32 exponential) with a zero V record; the output consists of a few positions of
+    the seventeenth that score 3 below it."""
+    say(f"wave attn best without values hd={hd} bands={bands} H={H} G={G} n={n} above={above}")
+    score, v_amp = np.full(n, -above), np.ones(n)
+    score[7 * 64 + 21], v_amp[7 * 64 + 21] = -0.5, 0.0
+    score[16 * 64 + 5:16 * 64 + 9] = -3.5
+    _run(hd, bands, H, H * G, score, v_amp, n_seq)
