@@ -174,7 +174,11 @@ int sp_hip_ship_decode(const sp_band_config_t *bc, const int *d_order, int vht2_
  * h / (n_q / n_heads_kv) (llama.cpp GQA grouping). Positions [0, n_kv) of
  * `layer` are attended. scores (optional): [n_q][n_kv] fp32 = kq_scale*q.K~.
  * out (optional): [n_q][head_dim] fp32 = softmax(scores) . V~.
- * Returns -1 for bad arguments or n_kv beyond the workspace sized at init. */
+ * Returns -1 for bad arguments or n_kv beyond the workspace sized at init.
+ * A cache has one workspace (partials and arrival counters) for the single-sequence calls and
+ * one for sp_hip_attn_decode_seqs: a single and a batched call may overlap on two streams, two
+ * calls of the same kind on one cache may not (the results of both are then undefined, and the
+ * counters they leave can spoil later calls). */
 int sp_hip_attn_decode(const sp_hip_cache_t *cc, int layer, int n_kv,
                        const float *d_q, int n_q, float kq_scale,
                        float *d_scores, float *d_out, void *stream);
@@ -217,7 +221,7 @@ size_t sp_hip_attn_noalloc_max_floats(void);
  * d_scores, sequence s's [n_q][seq_len[s]] block starting at element
  * n_q * (seq_len[0] + ... + seq_len[s-1]). Results equal n_seq separate calls over those
  * ranges. The matrix-core layouts (K 5/4/4 with V 5 at head_dim 64 and 96, K 5/5/4/3 with V 3
- * at head_dim 64, 128 and 256) run every sequence in one launch, in the workspace sized at
+ * at head_dim 64, 128 and 256) run every sequence in one launch, in a workspace sized at
  * init; other layouts run the general kernels once per sequence. */
 int sp_hip_attn_decode_seqs(const sp_hip_cache_t *cc, int layer, int n_seq, const int *seq_start,
                             const int *seq_len, const float *d_q, int n_q, float kq_scale, float *d_scores,

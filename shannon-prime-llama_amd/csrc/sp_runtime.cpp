@@ -432,7 +432,9 @@ extern "C" void sp_hip_band_dequantize(const void *d_input, float *d_output, con
 // ===========================================================================
 struct ShipPriv {
     SpPlan kplan, vplan;
-    float *ws = nullptr;
+    // attention workspaces, ws_floats each: the single-sequence calls', and the batched calls' own,
+    // so that a batched and a single call may overlap on two streams
+    float *ws = nullptr, *seq_ws = nullptr;
     size_t ws_floats = 0;
     int max_q = 0;
     // K coefficient-order calibration: fp64 sums of the fed vectors' transforms
@@ -521,9 +523,10 @@ extern "C" int sp_hip_cache_init(sp_hip_cache_t *cc, const sp_config_t *cfg, int
     if (ok) {
         pv->max_q = cfg->n_heads_kv * 8;
         pv->ws_floats = sp_attn_workspace_floats(pv->max_q, hd, max_seq_len);
-        ok = hip_ok(hipMalloc((void **)&pv->ws, pv->ws_floats * sizeof(float)), "hipMalloc attention workspace") &&
-             hip_ok(hipMemsetAsync(pv->ws, 0, pv->ws_floats * sizeof(float), (hipStream_t)stream),
-                    "attention workspace clear");  // the attention kernel's counters start at zero
+        for (float **w : {&pv->ws, &pv->seq_ws})
+            ok = ok && hip_ok(hipMalloc((void **)w, pv->ws_floats * sizeof(float)), "hipMalloc attention workspace") &&
+                 hip_ok(hipMemsetAsync(*w, 0, pv->ws_floats * sizeof(float), (hipStream_t)stream),
+                        "attention workspace clear");  // the attention kernel's counters start at zero
     }
     if (ok) ok = hip_ok(hipStreamSynchronize((hipStream_t)stream), "init sync");
     if (!ok) {
@@ -542,6 +545,7 @@ extern "C" void sp_hip_cache_free(sp_hip_cache_t *cc) {
     ShipPriv *pv = (ShipPriv *)cc->priv;
     if (pv) {
         if (pv->ws) (void)hipFree(pv->ws);
+        if (pv->seq_ws) (void)hipFree(pv->seq_ws);
         if (pv->stage_d) (void)hipFree(pv->stage_d);
         if (pv->stage_h) (void)hipHostFree(pv->stage_h);
         delete pv;
@@ -967,8 +971,8 @@ extern "C" int sp_hip_attn_decode_seqs(const sp_hip_cache_t *cc, int layer, int 
     ShipPriv *pv = (ShipPriv *)cc->priv;
     const hipStream_t s = (hipStream_t)(stream ? stream : cc->stream);
     if (n_q > pv->max_q) { set_err("attn seqs: n_q %d > %d", n_q, pv->max_q); return -1; }
-    // the matrix-core layouts: every sequence in one launch, in the cache's own workspace
-    const hipError_t we = sp_launch_attn_wave_ws(kp, vp, cc->d_mobius_order, A, T, pv->ws, pv->ws_floats, s);
+    // the matrix-core layouts: every sequence in one launch
+    const hipError_t we = sp_launch_attn_wave_ws(kp, vp, cc->d_mobius_order, A, T, pv->seq_ws, pv->ws_floats, s);
     if (we != hipErrorNotSupported) return hip_ok(we, "attn seqs") ? 0 : -1;
     // otherwise one single-sequence launch sequence per sequence, each over its range of records
     for (int i = 0; i < n_seq; i++) {
@@ -979,7 +983,7 @@ extern "C" int sp_hip_attn_decode_seqs(const sp_hip_cache_t *cc, int layer, int 
         Ai.q = d_q + (size_t)i * n_q * A.hd;
         Ai.scores = d_scores ? d_scores + T.soff[i] : nullptr;
         Ai.out = d_out ? d_out + (size_t)i * n_q * A.hd : nullptr;
-        if (!hip_ok(sp_launch_attn_decode(kp, vp, cc->d_mobius_order, Ai, pv->ws, pv->ws_floats, s), "attn seqs"))
+        if (!hip_ok(sp_launch_attn_decode(kp, vp, cc->d_mobius_order, Ai, pv->seq_ws, pv->ws_floats, s), "attn seqs"))
             return -1;
     }
     return 0;

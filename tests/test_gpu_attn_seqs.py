@@ -90,6 +90,42 @@ def test_ship_attention_seqs(hd, k_bits, v_bits, H, n_q, starts, lens, ms):
     cc.free()
 
 
+@pytest.mark.parametrize("hd,k_bits,v_bits", [(64, (5, 5, 4, 3), (3,)), (96, (5, 4, 4), (5,)), (128, (5, 5, 4, 3), (3,))])
+def test_batched_and_single_calls_on_two_streams(hd, k_bits, v_bits):
+    """Batched calls on one stream and single calls on another, over one cache and at the same
+    time, with several partials per KV head in both: the bits that each gives by itself."""
+    say(f"attn two streams hd={hd}")
+    H, n_q, ms, starts, lens = 8, 32, 8192, [0, 1500, 3000, 4], [3000, 1100, 5000, 8000]
+    side = [torch.cuda.Stream() for _ in range(2)]
+    cc = S.ShipCache(S.config(hd, 1, H, k_bits=k_bits, v_bits=v_bits), ms, stream=torch.cuda.current_stream().cuda_stream)
+    L, g = S.lib(), torch.Generator(device="cuda")
+    g.manual_seed(hd)
+    k, v = (torch.randn((ms, H * hd), generator=g, device="cuda").half() for _ in range(2))
+    S.check(L.sp_hip_write_layer(cc.ref, 0, 0, ms, p(k), p(v), H * hd, S.DTYPE_F16))
+    q = torch.randn((len(starts), n_q, hd), generator=g, device="cuda")
+    (_, sp_), (_, lp) = keep = _arr(starts), _arr(lens)
+    f = C.c_float(1.0 / math.sqrt(hd))
+
+    def batched(out, s):
+        S.check(L.sp_hip_attn_decode_seqs(cc.ref, 0, len(starts), sp_, lp, p(q), n_q, f, None, p(out), s))
+
+    def single(out, s):
+        S.check(L.sp_hip_attn_decode(cc.ref, 0, 7000, p(q), n_q, f, None, p(out), s))
+
+    alone = [empty_f32(q.numel()), empty_f32(n_q * hd)]
+    batched(alone[0], stream())
+    single(alone[1], stream())
+    outs = [[torch.zeros_like(a) for _ in range(40)] for a in alone]
+    torch.cuda.synchronize()
+    for a, b in zip(*outs):
+        batched(a, C.c_void_p(side[0].cuda_stream))
+        single(b, C.c_void_p(side[1].cuda_stream))
+    torch.cuda.synchronize()
+    for ref, got in zip(alone, outs):
+        assert all(torch.equal(ref.view(torch.int32), o.view(torch.int32)) for o in got)
+    cc.free()
+
+
 def test_sqfree_attention_seqs():
     """configs[3]'s geometry (skeleton 115, V one 3-bit band, GQA 8), four sequences of
     unequal length in one launch each of prep, split and merge."""
