@@ -21,8 +21,8 @@
 // decodes it (compile-time Knight CSR and record fields), the scores as dot products
 // with the prepared queries, an online softmax across the run's tiles, and the
 // weighted coefficient sums through LDS (the wave's coefficients transposed so that
-// each lane sums one coefficient over the tile's 64 positions); both products on the
-// matrix cores in fp32.
+// each lane sums one coefficient over the tile's 64 positions); both products in fp32, on
+// the matrix cores or (one or two query heads, on_matrix_cores()) on the vector unit.
 #include <cstdlib>
 #include <utility>
 
@@ -77,6 +77,18 @@ __device__ __forceinline__ f32x4 fma_heads(float a, float b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_4x4x1f32(a, b, c, CB, AB, 0);
 }
 
+// The vector unit's score factors of one query head in chunks of at most 16: the skeleton
+// part (SK factors) then the residual part (PAD - SK), a chunk never spanning both.
+template <int SK>
+struct QChunks {
+    static constexpr int NS = (SK + 15) / 16, NR = (PAD - SK + 15) / 16, N = NS + NR;
+    // coefficient index of chunk k's first factor, and the chunk's factor count
+    static constexpr int first(int k) { return k < NS ? 16 * k : SK + 16 * (k - NS); }
+    static constexpr int size(int k) {
+        return k < NS ? (SK - 16 * k < 16 ? SK - 16 * k : 16) : (PAD - SK - 16 * (k - NS) < 16 ? PAD - SK - 16 * (k - NS) : 16);
+    }
+};
+
 constexpr int NQ = (PAD + 15) / 16;  // registers of one head group's factors, 16 coefficients each
 
 // scores: s[g][C % 3][i](position) += q~[4g + i][C] * e[C](position), every C of the pack
@@ -129,8 +141,8 @@ __device__ __forceinline__ void sum_all(const float (&pw)[NG][NP], const float *
 }
 
 // LDS row pitch (floats) of the transposed coefficient chunk: 16-byte rows, eight lanes'
-// 16-byte pieces on distinct banks
-constexpr int EP = 68;
+// 16-byte pieces on distinct banks; for the vector unit's 4-byte reads, lanes on distinct banks
+constexpr int row_pitch(bool mx) { return mx ? 68 : 65; }
 
 // Scores, online softmax and the V records' weighted coefficient sums. Block
 // (kvh, run) takes tiles run, run + n_runs, ... of KV head kvh (64 positions each).
@@ -145,16 +157,16 @@ constexpr int EP = 68;
 // head i of the group, coefficient 16j + b) against the lane's own coefficients, in three
 // chains of sums; the weighted sums with the tile's weights (lane 4b + i of register j:
 // head i, position 16j + b) against the transposed chunk (lane = coefficient, four
-// positions per 16-byte LDS read).
+// positions per 16-byte LDS read). MX = false (one or two heads) takes the same sums on the
+// vector unit: the factors by scalar loads, the weights by LDS broadcasts.
 //
 // Bound by the decode of the two records (2400 vector instructions a tile beside 628
 // matrix instructions) and by latency at two waves per SIMD, which the 154 coefficients a
 // lane holds allow at most. Four sequences of 16384 over 4 KV heads and 8 query heads
-// each: 71 us with the products on the vector unit (4900 instructions a tile, queries and
-// weights by scalar loads and LDS broadcasts), 48 us now. Two chains of sums took 45 us and
+// each: 71 us with the products on the vector unit (4900 instructions a tile), 48 us here. Two chains of sums took 45 us and
 // four 50; the mean error against 64-bit results over 126 shapes was 4.6e-7 with two,
 // 3.9e-7 with three, 3.6e-7 with four, and 4.5e-7 before.
-template <int SK, class SLK, class SLV, int GM, bool OUT>
+template <int SK, class SLK, class SLV, int GM, bool MX, bool OUT>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2)))
 k_sqfree_attn_split(const unsigned char *__restrict__ kc0, const unsigned char *__restrict__ vc0, long long k_slot,
                     long long v_slot, const SpSeqTab T, int G, int hs, const float *__restrict__ prep0, int ps, int qo,
@@ -163,7 +175,9 @@ k_sqfree_attn_split(const unsigned char *__restrict__ kc0, const unsigned char *
     using GV = SqRec<PAD, SK, RBITS, true, SLV>;
     constexpr int NCK = RecTile<GK>::NCK > RecTile<GV>::NCK ? RecTile<GK>::NCK : RecTile<GV>::NCK;
     constexpr int C2 = PAD - 128;  // coefficients of the third 64-coefficient chunk
+    constexpr int EP = row_pitch(MX);
     constexpr int NG = (GM + 3) / 4;  // groups of four query heads
+    constexpr int PP = MX ? 4 * NG : GM;  // weights per position
     static_assert(C2 > 0 && C2 <= 32, "two whole chunks, and one of at most 32 coefficients");
     // the record stage and the transposed coefficient chunks share their memory: in
     // this one-wave block the stage's last reads (the V records) come before the first
@@ -172,7 +186,14 @@ k_sqfree_attn_split(const unsigned char *__restrict__ kc0, const unsigned char *
     __shared__ __attribute__((aligned(16))) float E[OUT ? 64 * EP : (NCK * 1024 + 16 + 3) / 4];
     static_assert(NCK * 1024 + 16 <= 64 * EP * 4, "the record stage fits the chunk memory");
     unsigned char *const stage = reinterpret_cast<unsigned char *>(E);
-    __shared__ __attribute__((aligned(16))) f32x4 Pw[OUT ? 64 * NG : 1];  // [position][group]
+    // At skeleton 77 the matrix instances stage a tile's V records beside its K records: held in
+    // registers through the K half they spilled there (52 to 63 dwords a lane, each load waited
+    // for and stored at once). 8 KV heads x 30000 positions, 4 query heads: 59.6 us against 52.0,
+    // 55.7 on the vector unit. At skeleton 115 (13 dwords) the registers are faster, 47.9 / 50.0.
+    constexpr bool V_STAGED = MX && SK == 77 && OUT;
+    unsigned char *const stage_v = V_STAGED ? stage + NCK * 1024 + 16 : stage;
+    static_assert(!V_STAGED || 2 * (NCK * 1024 + 16) <= 64 * EP * 4, "both sides' records fit the chunk memory");
+    __shared__ __attribute__((aligned(16))) float Pw[OUT ? 64 * PP : 4];  // [position][head]
     // block x: head group x (query heads x G .. x G + G - 1) of KV head x / hs
     const int hb = blockIdx.x, kvh = hb / hs, run = blockIdx.y, lane = threadIdx.x;
     // sequence blockIdx.z: its positions, prepared queries, score rows and partials
@@ -200,8 +221,15 @@ k_sqfree_attn_split(const unsigned char *__restrict__ kc0, const unsigned char *
     }
 #pragma unroll
     for (int g = 0; g < NG; g++) acc0[g] = acc1[g] = acc2[g] = z4;
+    float va0[GM], va1[GM], va2 = 0.0f;  // the vector unit's
+#pragma unroll
+    for (int h = 0; h < GM; h++) va0[h] = va1[h] = 0.0f;
     // third chunk: lane = coefficient 128 + c2i, positions 32 * half .. 32 * half + 31
-    // (the two halves are added at the end)
+    // (the two halves are added at the end). On the vector unit lane = coefficient 128 + vi of
+    // head vh, every position.
+    const int vi = lane % C2, vh = lane / C2;
+    const bool v_on = vh < GM;
+    static_assert(MX || GM <= 2, "a lane per head and coefficient of the third chunk");
     const int half = lane / 32, c2i = lane % 32 < C2 ? lane % 32 : C2 - 1;
 
     // a tile's K and V records load at the tile's start (holding the next tile's K records
@@ -209,17 +237,21 @@ k_sqfree_attn_split(const unsigned char *__restrict__ kc0, const unsigned char *
     // waves per SIMD; the other wave hides the load)
     for (int c = run; c < tpo; c += n_runs) {
         const int t = kvh * tpo + c;
+        // with the V records staged: an opaque copy of the lane index a tile, so that LDS
+        // addresses are not held through the loop either
+        int ln = lane;
+        if (V_STAGED) __asm__ volatile("" : "+v"(ln));
         RecTile<GK> Rk;
-        rec_tile_load<GK>(Rk, kc, k_slot, M, t, n_tiles, lane);
+        rec_tile_load<GK>(Rk, kc, k_slot, M, t, n_tiles, ln);
         RecTile<GV> Rv;
-        if (OUT) rec_tile_load<GV>(Rv, vc, v_slot, M, t, n_tiles, lane);
+        if (OUT) rec_tile_load<GV>(Rv, vc, v_slot, M, t, n_tiles, ln);
         // the head groups' factors, again for each tile (cache hits beside the records' loads):
         // held across the V half they cost the registers that keep it from spilling
         float q[NG][NQ];
         int zero = 0;
-        __asm__ volatile("" : "+v"(zero));  // no hoisting out of the tile loop
+        if constexpr (MX) __asm__ volatile("" : "+v"(zero));  // no hoisting out of the tile loop
 #pragma unroll
-        for (int g = 0; g < NG; g++) {
+        for (int g = 0; g < (MX ? NG : 0); g++) {
             // heads past the group's and coefficients past the pad repeat the last: their
             // products are never read
             const int h = 4 * g + li < G ? 4 * g + li : G - 1, o = h * ps + lb + zero;
@@ -233,10 +265,11 @@ k_sqfree_attn_split(const unsigned char *__restrict__ kc0, const unsigned char *
             }
         }
         __syncthreads();  // the previous tile is done with the stage
-        rec_tile_stage<GK>(Rk, stage, M, t, lane);
+        rec_tile_stage<GK>(Rk, stage, M, t, ln);
+        if (V_STAGED) rec_tile_stage<GV>(Rv, stage_v, M, t, ln);
         __syncthreads();
         uint32_t rk[GK::dwords];
-        rec_from_lds<GK>(rk, stage, lane);
+        rec_from_lds<GK>(rk, stage, ln);
         float e[PAD];
         sq_coefficients<SK, SLK>(rk, e);
         const int pos = c * 64 + lane;
@@ -244,15 +277,52 @@ k_sqfree_attn_split(const unsigned char *__restrict__ kc0, const unsigned char *
         f32x4 s3[NG][3];
 #pragma unroll
         for (int g = 0; g < NG; g++) s3[g][0] = s3[g][1] = s3[g][2] = z4;
-        score_all<NG>(q, e, s3, std::make_integer_sequence<int, PAD>{});
+        if constexpr (MX) score_all<NG>(q, e, s3, std::make_integer_sequence<int, PAD>{});
         float s[GM];
 #pragma unroll
         for (int h = 0; h < GM; h++) {
             s[h] = -INFINITY;
-            if (h < G && live) {
-                const f32x4(&v)[3] = s3[h / 4];
-                s[h] = (v[0][h % 4] + v[1][h % 4]) + v[2][h % 4];
-                if (scores) scores[(long long)(h0 + h) * s_stride + pos] = s[h];
+            if constexpr (MX) {
+                if (h < G && live) {
+                    const f32x4(&v)[3] = s3[h / 4];
+                    s[h] = (v[0][h % 4] + v[1][h % 4]) + v[2][h % 4];
+                    if (scores) scores[(long long)(h0 + h) * s_stride + pos] = s[h];
+                }
+            } else if (h < G) {
+                // the matrix path's sums bit for bit (three chains, coefficient k in chain k % 3)
+                // on the vector unit. The head's factors are wave-uniform and arrive by scalar
+                // loads, 16 at a time. With an output chunk k + 1 is loaded after the first product
+                // of chunk k (a scalar-load wait covers every scalar load in flight, so the next
+                // chunk cannot go out before the wait for the current one): 2% faster there; the
+                // scores-only instances measured 4% slower with it and keep the compiler's
+                // placement. (In a function of its own this spilled 130 scalar registers.)
+                const float *__restrict__ qh = pq + h * ps;
+                using QC = QChunks<SK>;
+                float qa[16], qb[16];
+#pragma unroll
+                for (int i = 0; i < QC::size(0); i++) qa[i] = qh[i];
+                float a[3] = {0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int k = 0; k < QC::N; k++) {
+                    float(&qc)[16] = (k & 1) ? qb : qa;
+                    float(&qn)[16] = (k & 1) ? qa : qb;
+                    const int e0 = QC::first(k);
+                    a[e0 % 3] = fmaf(qc[0], e[e0], a[e0 % 3]);
+                    if (k + 1 < QC::N) {
+                        const float *__restrict__ qs = qh + (k + 1 < QC::NS ? 16 * (k + 1) : qo + 16 * (k + 1 - QC::NS));
+                        if constexpr (OUT) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                        for (int i = 0; i < QC::size(k + 1); i++) qn[i] = qs[i];
+                        if constexpr (OUT) __builtin_amdgcn_sched_barrier(0);
+                    }
+#pragma unroll
+                    for (int i = 1; i < QC::size(k); i++) a[(e0 + i) % 3] = fmaf(qc[i], e[e0 + i], a[(e0 + i) % 3]);
+                }
+                const float v = (a[0] + a[1]) + a[2];
+                if (live) {
+                    s[h] = v;
+                    if (scores) scores[(long long)(h0 + h) * s_stride + pos] = v;
+                }
             }
         }
         if (!OUT) continue;
@@ -273,14 +343,21 @@ k_sqfree_attn_split(const unsigned char *__restrict__ kc0, const unsigned char *
                 pr[h / 4][h % 4] = p;
             }
         }
+        if constexpr (MX) {
 #pragma unroll
-        for (int g = 0; g < NG; g++) Pw[lane * NG + g] = pr[g];
+            for (int g = 0; g < NG; g++) *reinterpret_cast<f32x4 *>(Pw + ln * PP + 4 * g) = pr[g];
+        } else {
+#pragma unroll
+            for (int h = 0; h < GM; h++) Pw[ln * PP + h] = pr[0][h];
+        }
         // ---- V records of the tile, then their coefficients ----
         __syncthreads();  // every lane has read its K record from the stage
-        rec_tile_stage<GV>(Rv, stage, M, t, lane);
-        __syncthreads();
+        if (!V_STAGED) {
+            rec_tile_stage<GV>(Rv, stage, M, t, ln);
+            __syncthreads();
+        }
         uint32_t rv[GV::dwords];
-        rec_from_lds<GV>(rv, stage, lane);
+        rec_from_lds<GV>(rv, stage_v, ln);
         float ev[PAD];
         sq_coefficients<SK, SLV>(rv, ev);
 #pragma unroll
@@ -288,33 +365,50 @@ k_sqfree_attn_split(const unsigned char *__restrict__ kc0, const unsigned char *
             acc0[h / 4][h % 4] *= alpha[h];
             acc1[h / 4][h % 4] *= alpha[h];
             acc2[h / 4][h % 4] *= alpha[h];
+            va0[h] *= alpha[h];
+            va1[h] *= alpha[h];
+            if (h == vh) va2 *= alpha[h];
         }
         // ---- weighted coefficient sums: chunk of 64 coefficients transposed through
         // LDS (row = coefficient, column = position), lane = coefficient ----
-        const float *const pf = reinterpret_cast<const float *>(Pw);
         float pw[NG][4];  // lane 4b + i, register j: head i, position 16j + b
+        if constexpr (MX) {
 #pragma unroll
-        for (int g = 0; g < NG; g++)
+            for (int g = 0; g < NG; g++)
 #pragma unroll
-            for (int j = 0; j < 4; j++) pw[g][j] = pf[(16 * j + lb) * (4 * NG) + 4 * g + li];
+                for (int j = 0; j < 4; j++) pw[g][j] = Pw[(16 * j + lb) * PP + 4 * g + li];
+        }
 #pragma unroll
         for (int ch = 0; ch < 3; ch++) {
             const int i0 = 64 * ch, n_i = ch < 2 ? 64 : C2;
 #pragma unroll
             for (int i = 0; i < 64; i++)
-                if (i < n_i) E[i * EP + lane] = ev[i0 + i];
+                if (i < n_i) E[i * EP + ln] = ev[i0 + i];
             __syncthreads();
-            if (ch == 0) {
-                sum_all<NG, 16, 4, 4>(pw, E + lane * EP, acc0);
+            if constexpr (!MX) {
+                if (ch < 2) {
+                    float(&va)[GM] = ch == 0 ? va0 : va1;
+#pragma unroll 4
+                    for (int p = 0; p < 64; p++) {
+                        const float ei = E[ln * EP + p];
+#pragma unroll
+                        for (int h = 0; h < GM; h++) va[h] = fmaf(Pw[p * PP + h], ei, va[h]);
+                    }
+                } else if (v_on) {
+#pragma unroll 4
+                    for (int p = 0; p < 64; p++) va2 = fmaf(Pw[p * PP + vh], E[vi * EP + p], va2);
+                }
+            } else if (ch == 0) {
+                sum_all<NG, 16, 4, 4>(pw, E + ln * EP, acc0);
             } else if (ch == 1) {
-                sum_all<NG, 16, 4, 4>(pw, E + lane * EP, acc1);
+                sum_all<NG, 16, 4, 4>(pw, E + ln * EP, acc1);
             } else {
                 // half h of the wave: head i, position 32h + 8j + b of its eight blocks b
 #pragma unroll
                 for (int g = 0; g < NG; g++)
 #pragma unroll
                     for (int j = 0; j < 4; j++)
-                        pw[g][j] = pf[(32 * half + 8 * j + lb % 8) * (4 * NG) + 4 * g + li];
+                        pw[g][j] = Pw[(32 * half + 8 * j + lb % 8) * PP + 4 * g + li];
                 sum_all<NG, 8, 3, 2>(pw, E + c2i * EP + 32 * half, acc2);
             }
             __syncthreads();
@@ -324,7 +418,8 @@ k_sqfree_attn_split(const unsigned char *__restrict__ kc0, const unsigned char *
     // ---- the run's partial per query head ----
 #pragma unroll
     for (int h = 0; h < GM; h++) {
-        const float a2 = acc2[h / 4][h % 4] + __shfl_xor(acc2[h / 4][h % 4], 32);
+        float a2 = 0.0f;
+        if constexpr (MX) a2 = acc2[h / 4][h % 4] + __shfl_xor(acc2[h / 4][h % 4], 32);
         if (h >= G) continue;
         float *dst = part + ((long long)(h0 + h) * n_runs + run) * pp;
         if (lane == 0) {
@@ -333,9 +428,10 @@ k_sqfree_attn_split(const unsigned char *__restrict__ kc0, const unsigned char *
             dst[2] = 0.0f;
             dst[3] = 0.0f;
         }
-        dst[4 + lane] = acc0[h / 4][h % 4];
-        dst[4 + 64 + lane] = acc1[h / 4][h % 4];
-        if (lane < C2) dst[4 + 128 + lane] = a2;
+        dst[4 + lane] = MX ? acc0[h / 4][h % 4] : va0[h];
+        dst[4 + 64 + lane] = MX ? acc1[h / 4][h % 4] : va1[h];
+        if (MX && lane < C2) dst[4 + 128 + lane] = a2;
+        if (!MX && h == vh) dst[4 + 128 + vi] = va2;
     }
 }
 
@@ -343,17 +439,37 @@ using SkelL77 = Layout<77, 5, 4, 4, 4, 5>;
 using SkelL115 = Layout<115, 5, 4, 4, 4, 5>;
 using SkelL115V3 = Layout<115, 3>;
 
+// compute units of the current device (256 when the runtime cannot say)
+int device_cus() {
+    int dev = 0, n = 0;
+    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+        n <= 0)
+        n = 256;
+    return n;
+}
+
+// Whether a launch over `tiles` tiles (all sequences, KV heads and head groups) for g query heads
+// a block takes its products on the matrix cores. A matrix instruction serves four heads
+// whatever the number used, in the time of two vector instructions, and needs no factors from
+// scalar loads: the better one for three heads and more, and for one or two while a SIMD has
+// few waves to hide those loads (one wave a SIMD for one head, two for two). Measured on
+// 256 CUs, 8 KV heads, skeleton 115, us, vector / matrix: one head, 30000 positions (3752 tiles)
+// 38.3 / 46.2, 16 sequences of up to 1500 (about 2000) 35.8 / 39.2, 4 of up to 4000 (1300) 28.2 /
+// 31.1, 2 KV heads at 30000 (938) 31.2 / 29.9; two heads, 43.2 / 47.0, 40.9 / 40.4, 32.7 / 31.9;
+// four heads at 30000 52.9 / 48.1. Both give the same scores bit for bit.
+bool on_matrix_cores(int g, long long tiles) { return g > 2 || tiles <= 4LL * g * device_cus(); }
+
 // hs head groups per KV head (1 or 2): block x takes the query heads of group x.
-template <int SK, class SLK, class SLV, int GM>
+template <int SK, class SLK, class SLV, int GM, bool MX>
 void launch_split(const SpSqAttnArgs &A, const SpSeqTab &T, const float *prep, float *part, int n_runs, int hs,
                   hipStream_t s) {
     const dim3 grid(A.n_kvh * hs, n_runs, T.n_seq), block(64);
     const int G = A.n_q / A.n_kvh / hs;
     if (A.out)
-        hipLaunchKernelGGL((k_sqfree_attn_split<SK, SLK, SLV, GM, true>), grid, block, 0, s, A.kcache, A.vcache,
+        hipLaunchKernelGGL((k_sqfree_attn_split<SK, SLK, SLV, GM, MX, true>), grid, block, 0, s, A.kcache, A.vcache,
                            A.k_slot_bytes, A.v_slot_bytes, T, G, hs, prep, A.ps, A.qo, A.scores, part, A.pp, n_runs);
     else
-        hipLaunchKernelGGL((k_sqfree_attn_split<SK, SLK, SLV, GM, false>), grid, block, 0, s, A.kcache, A.vcache,
+        hipLaunchKernelGGL((k_sqfree_attn_split<SK, SLK, SLV, GM, MX, false>), grid, block, 0, s, A.kcache, A.vcache,
                            A.k_slot_bytes, A.v_slot_bytes, T, G, hs, prep, A.ps, A.qo, A.scores, part, A.pp, n_runs);
 }
 
@@ -361,10 +477,14 @@ template <int SK, class SLK, class SLV>
 void launch_split_g(const SpSqAttnArgs &A, const SpSeqTab &T, const float *prep, float *part, int n_runs, int hs,
                     hipStream_t s) {
     const int G = A.n_q / A.n_kvh / hs;
-    if (G <= 1) launch_split<SK, SLK, SLV, 1>(A, T, prep, part, n_runs, hs, s);
-    else if (G <= 2) launch_split<SK, SLK, SLV, 2>(A, T, prep, part, n_runs, hs, s);
-    else if (G <= 4) launch_split<SK, SLK, SLV, 4>(A, T, prep, part, n_runs, hs, s);
-    else launch_split<SK, SLK, SLV, 8>(A, T, prep, part, n_runs, hs, s);
+    long long tiles = 0;
+    for (int i = 0; i < T.n_seq; i++) tiles += (long long)A.n_kvh * hs * ((T.len[i] + 63) / 64);
+    const bool mx = on_matrix_cores(G, tiles);
+    if (G <= 1 && !mx) launch_split<SK, SLK, SLV, 1, false>(A, T, prep, part, n_runs, hs, s);
+    else if (G <= 2 && !mx) launch_split<SK, SLK, SLV, 2, false>(A, T, prep, part, n_runs, hs, s);
+    else if (G <= 2) launch_split<SK, SLK, SLV, 2, true>(A, T, prep, part, n_runs, hs, s);
+    else if (G <= 4) launch_split<SK, SLK, SLV, 4, true>(A, T, prep, part, n_runs, hs, s);
+    else launch_split<SK, SLK, SLV, 8, true>(A, T, prep, part, n_runs, hs, s);
 }
 
 template <class SL>
@@ -393,19 +513,10 @@ template <int SK, class SLK, class SLV, int GM>
 int resident_per_cu(bool out) {
     int nb = 0;
     const hipError_t e =
-        out ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_sqfree_attn_split<SK, SLK, SLV, GM, true>, 64, 0)
-            : hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_sqfree_attn_split<SK, SLK, SLV, GM, false>, 64, 0);
+        out ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_sqfree_attn_split<SK, SLK, SLV, GM, (GM > 2), true>, 64, 0)
+            : hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_sqfree_attn_split<SK, SLK, SLV, GM, (GM > 2), false>, 64, 0);
     return e == hipSuccess && nb > 0 ? nb : 4;
 }
-// compute units of the current device (256 when the runtime cannot say)
-int device_cus() {
-    int dev = 0, n = 0;
-    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        n <= 0)
-        n = 256;
-    return n;
-}
-
 template <int SK, class SLK, class SLV>
 int resident_per_cu_g(int G, bool out) {
     if (G <= 1) return resident_per_cu<SK, SLK, SLV, 1>(out);
