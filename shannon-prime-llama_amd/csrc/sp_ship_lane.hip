@@ -108,14 +108,16 @@ __device__ __forceinline__ void enc_tile(const uint4 (&in)[row_bytes<DT>(LY::hd)
 // arithmetic, two waves fit per SIMD and one's loads overlap the other's work.
 // The record stage reuses the row buffer once the rows are in registers: 17 KB
 // per single-wave block lets two waves share each SIMD.
-template <class LY, int DT, int NORM, bool MOB>
+// SIDES: the calls that the grid is shared by. (The grid's size is read behind the first tile:
+// read before it, its own cache line adds 0.2 us to every call.)
+template <class LY, int DT, int NORM, bool MOB, int SIDES>
 __device__ __forceinline__ void enc_tiles(const void *src, long long so, long long si, unsigned char *dst,
-                                          long long dout, const TileMap &M, int t, int step, int n_tiles,
+                                          long long dout, const TileMap &M, int t, int n_tiles,
                                           const XfConst &K, unsigned char *rows) {
     constexpr int RB = row_bytes<DT>(LY::hd), RP = RB + 16, CPR = RB / 16, B = LY::total, DW = LY::dwords;
     static_assert(64 * B + 16 <= 64 * RP, "record stage must fit in the row buffer");
     const int lane = threadIdx.x;
-    for (; t < n_tiles; t += step) {
+    for (; t < n_tiles; t += (int)gridDim.x / SIDES) {
         uint4 in[CPR];
         tile_rows_in<DT, LY::hd>(src, so, si, M, t, lane, rows, in);
         uint32_t rec[DW];
@@ -130,8 +132,8 @@ k_ship_encode_lane(const void *__restrict__ src, long long so, long long si,
                    unsigned char *__restrict__ dst, long long dout, int n_inner, int tiles_per_outer,
                    int n_tiles, const XfConst K) {
     __shared__ __attribute__((aligned(16))) unsigned char rows[64 * (row_bytes<DT>(LY::hd) + 16)];
-    enc_tiles<LY, DT, NORM, MOB>(src, so, si, dst, dout, TileMap{tiles_per_outer, n_inner}, blockIdx.x, gridDim.x,
-                                 n_tiles, K, rows);
+    enc_tiles<LY, DT, NORM, MOB, 1>(src, so, si, dst, dout, TileMap{tiles_per_outer, n_inner}, blockIdx.x, n_tiles, K,
+                                    rows);
 }
 
 // K and V of one call in one launch: the first half of the grid walks K's tiles,
@@ -147,8 +149,8 @@ k_ship_encode_lane_kv(const void *__restrict__ src_k, const void *__restrict__ s
     __shared__ __attribute__((aligned(16))) unsigned char rows[64 * (row_bytes<DT>(LK::hd) + 16)];
     const int nb = gridDim.x / 2, b = blockIdx.x;
     const TileMap M{tiles_per_outer, n_inner};
-    if (b < nb) enc_tiles<LK, DT, 0, true>(src_k, so, si, dst_k, dout_k, M, b, nb, n_tiles, K, rows);
-    else enc_tiles<LV, DT, 0, false>(src_v, so, si, dst_v, dout_v, M, b - nb, nb, n_tiles, K, rows);
+    if (b < nb) enc_tiles<LK, DT, 0, true, 2>(src_k, so, si, dst_k, dout_k, M, b, n_tiles, K, rows);
+    else enc_tiles<LV, DT, 0, false, 2>(src_v, so, si, dst_v, dout_v, M, b - nb, n_tiles, K, rows);
 }
 
 // ---------------------------------------------------------------------------
@@ -470,6 +472,19 @@ hipError_t dec_dispatch(const SpPlan &P, bool mob, const unsigned char *src, lon
     return hipErrorNotSupported;
 }
 
+// Whether a run of records off a dword (which the general kernels take as well) is faster here.
+// Not where fp32 rows fill the LDS so far that a CU holds four blocks (head_dim 128) or two
+// (256): past one round of those the general kernels' many waves are faster. 8 heads, V
+// records from cell 1, general / here, us: head_dim 128 read 13.4 / 10.2 at 1024 tiles, 19.6 / 22.0 at
+// 2048, 32.3 / 37.8 at 4096 (written 44.4 / 31.2); head_dim 256 written 18.1 / 13.4 at 512, 22.1 / 26.0
+// at 752, 98 / 105 at 4096, read 16.8 / 15.8, 19.7 / 27.5, 79 / 105. Reads of head_dim 256 up to
+// half a tile per CU take 11.9 / 12.6.
+bool off_dword_pays(int dtype, int hd, bool decode, long long tiles) {
+    if (dtype == SP_DT_F16 || hd < 128 || (hd == 128 && !decode)) return true;
+    const long long cus = device_cu_count(), round = cus * (160 * 1024 / (64 * (4 * hd + 16)));
+    return tiles <= round && !(decode && hd == 256 && 2 * tiles <= cus);
+}
+
 }  // namespace
 
 // Returns hipErrorNotSupported (nothing launched) when no specialization fits:
@@ -479,13 +494,16 @@ hipError_t dec_dispatch(const SpPlan &P, bool mob, const unsigned char *src, lon
 // accesses, which the hardware takes at any alignment, and one 2-byte access per
 // lane for the rest of an even-sized record run. So a run from an odd cell of 42-,
 // 50-, 58- or 62-byte records stays here (8 heads x 2048 tokens of head_dim 96 from
-// cell 1: encode 44 us on the general kernel, 7.9 here; 7.7 from cell 0).
+// cell 1: encode 44 us on the general kernel, 7.9 here; 7.7 from cell 0), up to the
+// sizes of off_dword_pays().
 hipError_t sp_launch_ship_encode_lane(const SpPlan &P, bool default_order, const void *src, int dtype,
                                       long long so, long long si, unsigned char *dst, long long dout,
                                       int n_outer, int n_inner, hipStream_t s) {
     const int esz = dtype == SP_DT_F16 ? 2 : 4;
     if (((uintptr_t)src % 16) || ((so * esz) % 16) || ((si * esz) % 16)) return hipErrorNotSupported;
     if (((uintptr_t)dst % 2) || (dout % 2)) return hipErrorNotSupported;
+    if ((((uintptr_t)dst % 4) || (dout % 4)) && !off_dword_pays(dtype, P.hd, false, kv_tiles(n_outer, n_inner)))
+        return hipErrorNotSupported;
     if (dtype == SP_DT_F16) return enc_dispatch<SP_DT_F16>(P, default_order, src, so, si, dst, dout, n_outer, n_inner, s);
     return enc_dispatch<SP_DT_F32>(P, default_order, src, so, si, dst, dout, n_outer, n_inner, s);
 }
@@ -496,6 +514,8 @@ hipError_t sp_launch_ship_decode_lane(const SpPlan &P, bool default_order, const
     const int esz = dtype == SP_DT_F16 ? 2 : 4;
     if (((uintptr_t)dst % 16) || ((dout * esz) % 16) || ((din * esz) % 16)) return hipErrorNotSupported;
     if (((uintptr_t)src % 2) || (so % 2)) return hipErrorNotSupported;
+    if ((((uintptr_t)src % 4) || (so % 4)) && !off_dword_pays(dtype, P.hd, true, kv_tiles(n_outer, n_inner)))
+        return hipErrorNotSupported;
     if (dtype == SP_DT_F16) return dec_dispatch<SP_DT_F16>(P, default_order, src, so, dst, dout, din, n_outer, n_inner, s);
     return dec_dispatch<SP_DT_F32>(P, default_order, src, so, dst, dout, din, n_outer, n_inner, s);
 }
@@ -533,6 +553,11 @@ hipError_t sp_launch_ship_decode_lane_kv(const SpPlan &KP, const SpPlan &VP, con
         return hipErrorNotSupported;
     if (((uintptr_t)dst_k % 16) || ((uintptr_t)dst_v % 16) || ((dout * esz) % 16) || ((din * esz) % 16) ||
         ((uintptr_t)src_k % 2) || ((uintptr_t)src_v % 2) || (so_k % 2) || (so_v % 2))
+        return hipErrorNotSupported;
+    // fp32 rows of head_dim 256 with V records off a dword: V on the general kernels (see
+    // off_dword_pays), 8 heads, us, apart / merged: 51.4 / 51.1 at 1024 tiles a side, 94 / 104 at 2048
+    if (dtype != SP_DT_F16 && VP.hd == 256 && (((uintptr_t)src_v % 4) || (so_v % 4)) &&
+        kv_tiles(n_outer, n_inner) > 4LL * device_cu_count())
         return hipErrorNotSupported;
 #define SP_TRY(LK, LV)                                                                                              \
     if (layout_matches<LK>(KP) && layout_matches<LV>(VP))                                                           \

@@ -151,3 +151,32 @@ def test_sides_read_into_one_buffer(kind):
     assert torch.equal(mixed[:, 0], ref[0]) and torch.equal(mixed[:, 1], ref[1])
     assert torch.equal(one, ref[1]) and not torch.equal(ref[0], ref[1])
     cc.free()
+
+
+@pytest.mark.parametrize("hd,n", [(128, 8300), (256, 4200)])
+def test_large_fp32_runs_off_a_dword(hd, n):
+    """8 heads of fp32 rows from cell 1 (V records off a dword) past one round of the lane kernels'
+    blocks on 256 CUs, where the general kernels take them, K and V and V alone, against the
+    same rows in calls of 1000 (the lane kernels)."""
+    H = 8
+    say(f"lane cells large fp32 hd={hd} n={n}")
+    g = torch.Generator(device="cuda")
+    g.manual_seed(hd)
+    x = [torch.randn((n, H * hd), generator=g, device="cuda") for _ in range(2)]
+    st = torch.cuda.current_stream().cuda_stream
+    whole, parts = (S.ShipCache(S.config(hd, 1, H), n + 2, stream=st) for _ in range(2))
+    L, B = S.lib(), [whole.c.k_bands.total_bytes, whole.c.v_bands.total_bytes]
+    y = [torch.zeros_like(x[0]) for _ in range(5)]
+    S.check(L.sp_hip_write_layer(whole.ref, 0, 1, n, p(x[0]), p(x[1]), H * hd, S.DTYPE_F32))
+    S.check(L.sp_hip_read_layer(whole.ref, 0, 1, n, p(y[0]), p(y[1]), H * hd, S.DTYPE_F32, -1))
+    S.check(L.sp_hip_read_layer(whole.ref, 0, 1, n, None, p(y[4]), H * hd, S.DTYPE_F32, -1))
+    for a in range(0, n, 1000):
+        m = min(1000, n - a)
+        S.check(L.sp_hip_write_layer(parts.ref, 0, 1 + a, m, p(x[0][a:]), p(x[1][a:]), H * hd, S.DTYPE_F32))
+        S.check(L.sp_hip_read_layer(parts.ref, 0, 1 + a, m, p(y[2][a:]), p(y[3][a:]), H * hd, S.DTYPE_F32, -1))
+    for a, b in zip(_records(whole, B, H, n + 2), _records(parts, B, H, n + 2)):
+        np.testing.assert_array_equal(a, b)
+    for a, b in ((0, 2), (1, 3), (4, 3)):
+        assert torch.equal(y[a].view(torch.int32), y[b].view(torch.int32))
+    whole.free()
+    parts.free()
