@@ -470,7 +470,10 @@ constexpr int wave_waves_per_simd(int hd, int nh, bool multi) {
     return hd == 256 ? 2 : multi && (hd == 128 || nh == 2) ? 3 : 4;
 }
 // The launch shapes that exist: blocks of 4, 8 or 16 waves at one tile per wave; several
-// tiles per wave in blocks of up to that many waves (0: none).
+// tiles per wave in blocks of up to that many waves (0: none; 5 to 8 heads at head_dim 128, us
+// at one tile per wave in blocks of 16 / the best with several: 8 KV heads x 60000 positions
+// 38.8 / 66.5, x 131000 77.5 / 122.7), and in blocks of 16 for the scores alone of one
+// sequence at head_dim 128.
 constexpr int wave_max_nw(int hd) { return hd == 256 ? 8 : 16; }
 constexpr int wave_multi_nw(int hd, int nh) {
     return hd == 256 ? 8 : hd == 128 ? (nh == 1 ? 4 : 0) : nh == 1 ? 16 : 4;
@@ -486,7 +489,7 @@ constexpr int wave_multi_nw(int hd, int nh) {
 // scale (a finite sum times 0 adds exactly nothing, so the scores and outputs
 // equal those with the bands read as 0, at the cost of the all-band loop).
 template <class LY, int NW, bool WANT_OUT, int NH, bool MULTI, bool SEQS>
-__global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(wave_waves_per_simd(LY::HD, NH, MULTI))))
+__global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(wave_waves_per_simd(LY::HD, NH, MULTI && NW < 16))))
 k_attn_wave(const SpAttnArgs A, const int *__restrict__ order, float *__restrict__ part, int part_rows, int tpw, int kbands,
             int vbands, int *__restrict__ counters, const std::conditional_t<SEQS, SpSeqTab, SpNoTab> T) {
     using L = WaveLds<LY, NW>;
@@ -1061,17 +1064,23 @@ k_attn_wave(const SpAttnArgs A, const int *__restrict__ order, float *__restrict
 }
 
 template <class LY, int NW, int NH, bool MULTI, bool SEQS>
-void launch_wave(const SpAttnArgs &A, const SpSeqTab &T, const int *order, float *part, int nb, int tpw, int kb_lim,
+hipError_t launch_wave(const SpAttnArgs &A, const SpSeqTab &T, const int *order, float *part, int nb, int tpw, int kb_lim,
                  int vb_lim, int *cnt, hipStream_t s) {
     const dim3 grid(A.n_kvh, nb, T.n_seq), block(64 * NW);
     std::conditional_t<SEQS, SpSeqTab, SpNoTab> tab{};
     if constexpr (SEQS) tab = T;
-    if (A.out)
-        hipLaunchKernelGGL((k_attn_wave<LY, NW, true, NH, MULTI, SEQS>), grid, block, 0, s, A, order, part, nb, tpw, kb_lim,
-                           vb_lim, cnt, tab);
-    else
-        hipLaunchKernelGGL((k_attn_wave<LY, NW, false, NH, MULTI, SEQS>), grid, block, 0, s, A, order, part, nb, tpw, kb_lim,
-                           vb_lim, cnt, tab);
+    if constexpr (!MULTI || NW <= wave_multi_nw(LY::HD, NH)) {
+        if (A.out) {
+            hipLaunchKernelGGL((k_attn_wave<LY, NW, true, NH, MULTI, SEQS>), grid, block, 0, s, A, order, part, nb, tpw, kb_lim,
+                               vb_lim, cnt, tab);
+            return hipGetLastError();
+        }
+    } else if (A.out) {
+        return hipErrorInvalidValue;
+    }
+    hipLaunchKernelGGL((k_attn_wave<LY, NW, false, NH, MULTI, SEQS>), grid, block, 0, s, A, order, part, nb, tpw, kb_lim,
+                       vb_lim, cnt, tab);
+    return hipGetLastError();
 }
 
 // Whether the K and V plans are the layout's records.
@@ -1118,18 +1127,20 @@ using WaveHd128 = WaveLayout<128, 3, false, 5, 5, 4, 3>;
 using WaveHd256 = WaveLayout<256, 3, true, 5, 5, 4, 3>;
 
 template <class LY, int NW, int NH, bool MULTI>
-void launch_wave_seqs(const SpWaveLaunch &W) {
+hipError_t launch_wave_seqs(const SpWaveLaunch &W) {
     if (W.T.n_seq > 1)
-        launch_wave<LY, NW, NH, MULTI, true>(W.A, W.T, W.order, W.part, W.nb, W.tpw, W.kbands, W.vbands, W.counters, W.s);
-    else
-        launch_wave<LY, NW, NH, MULTI, false>(W.A, W.T, W.order, W.part, W.nb, W.tpw, W.kbands, W.vbands, W.counters, W.s);
+        return launch_wave<LY, NW, NH, MULTI, true>(W.A, W.T, W.order, W.part, W.nb, W.tpw, W.kbands, W.vbands, W.counters, W.s);
+    return launch_wave<LY, NW, NH, MULTI, false>(W.A, W.T, W.order, W.part, W.nb, W.tpw, W.kbands, W.vbands, W.counters, W.s);
 }
 template <class LY, int NW, int NH>
 hipError_t wave_launch_nw(const SpWaveLaunch &W) {
-    if (W.tpw == 1) launch_wave_seqs<LY, NW, NH, false>(W);
-    else if constexpr (NW <= wave_multi_nw(LY::HD, NH)) launch_wave_seqs<LY, NW, NH, true>(W);
-    else return hipErrorInvalidValue;
-    return hipGetLastError();
+    if (W.tpw == 1) return launch_wave_seqs<LY, NW, NH, false>(W);
+    if constexpr (NW <= wave_multi_nw(LY::HD, NH)) return launch_wave_seqs<LY, NW, NH, true>(W);
+    else if constexpr (LY::HD == 128 && NW == 16) {  // scores of one sequence
+        if (W.T.n_seq == 1)
+            return launch_wave<LY, NW, NH, true, false>(W.A, W.T, W.order, W.part, W.nb, W.tpw, W.kbands, W.vbands, W.counters, W.s);
+    }
+    return hipErrorInvalidValue;
 }
 template <class LY, int NH>
 hipError_t wave_launch_nh(const SpWaveLaunch &W) {

@@ -32,16 +32,27 @@ static int wave_device_cus() {
 //   * where several tiles per wave need 168 registers (3 waves a SIMD, blocks of 4), from 1.5
 //     times the wave slots on, aimed at two blocks a CU (more only add partials) and at most 8
 //     tiles (head_dim 128: 8192 tiles 26.5 us against 29.0 at one tile per wave, 16384 tiles
-//     39.1 against 54.1, 4096 tiles 18.7 against 16.3).
+//     39.1 against 54.1, 4096 tiles 18.7 against 16.3). One sequence's scores alone, with no
+//     partials to merge, go in blocks of 16 over one round there, from 9/8 of the slots on (60000
+//     positions 9.3 us against 11.5, 131000 17.8 against 20.6, 40000 9.0 against 10.6, 33000, below the
+//     line, 9.0 against 8.5; 8 query heads 15.0 against 16.5, 31.3 against 33.5).
+// The block sizes' lines were measured at head_dim 128; at 64, 96 and 256, 1 to 8 query heads and
+// one sequence of 250 to 40000 positions they are within 10% of the best of the three sizes but
+// for 5000 tiles at one tile per wave (8 waves would be 15-25% faster than 16). Batches of
+// short sequences with 5 to 8 heads per KV head would be up to twice as fast in blocks of 16
+// (12 of up to 600 positions: 25.9 us, 12.2): the last block's merge is a round per block's threads.
 struct WaveShape {
     int nw, tpw;
 };
-static WaveShape wave_shape(int hd, int nh, int cus, long long tiles, long long longest) {
+static WaveShape wave_shape(int hd, int nh, int cus, long long tiles, long long longest, int n_seq, bool out) {
     const int most = wave_max_nw(hd), multi = wave_multi_nw(hd, nh);
     const long long slots = (long long)cus * 4 * wave_waves_per_simd(hd, nh, false);
     // (5 to 8 tiles: one block of 8 has no partials to merge, 7.8 us against 9.2 at 333 positions)
     WaveShape s = {longest <= 4 ? 4 : longest <= 8 ? 8 : longest <= 64 ? 4 : longest <= 256 ? 8 : most, 1};
-    if (multi == 4 && 2 * tiles >= 3 * slots) {
+    if (hd == 128 && !out && n_seq == 1 && 8 * tiles >= 9 * slots) {
+        s.nw = 16;
+        s.tpw = (int)((tiles + slots - 1) / slots);
+    } else if (multi == 4 && 2 * tiles >= 3 * slots) {
         s.nw = 4;
         s.tpw = (int)std::min({8LL, (tiles + slots / 2 - 1) / (slots / 2), (longest + 3) / 4});
     } else if (multi > 4 && tiles >= slots) {
@@ -84,7 +95,7 @@ hipError_t sp_launch_attn_wave(const SpPlan &KP, const SpPlan &VP, const int *or
                 tiles += A.n_kvh * t;
                 longest = std::max(longest, t);
             }
-            sh = wave_shape(A.hd, nh, cus, tiles, longest);
+            sh = wave_shape(A.hd, nh, cus, tiles, longest, n, A.out != nullptr);
             nb = (int)((longest + (long long)sh.nw * sh.tpw - 1) / ((long long)sh.nw * sh.tpw));
             if (!A.out || n == 1 || nb == 1 ||
                 (n * A.n_kvh <= SP_ATTN_MAX_KVH && (size_t)n * A.n_q * nb * (A.hd + 2) <= part_floats))

@@ -47,8 +47,8 @@ ATTN_CASES = [
     (4, 4, 256, 128, False),     # MHA, exactly one split, no Mobius
     (16, 2, 4099, 128, True),    # GQA 8, 17 splits, a 3-position last tile
     (3, 3, 1, 128, True),        # a single position
-    (16, 8, 777, 256, True),     # Gemma-3 head_dim (general kernel)
-    (8, 8, 129, 64, True),       # general kernel
+    (16, 8, 777, 256, True),     # Gemma-3 head_dim
+    (8, 8, 129, 64, True),
     (12, 4, 700, 128, True),     # GQA 3: one unused head column of the score matrix cores
     (20, 4, 333, 128, True),     # GQA 5: a second column set, three of its heads unused
 ]
@@ -57,19 +57,15 @@ ATTN_CASES = [
 def general_kernel_only(monkeypatch):
     """Route decode attention to the general kernel (sp_attn.hip's split kernel)."""
     monkeypatch.setenv("SP_HIP_NO_MFMA_ATTN", "1")
-    monkeypatch.setenv("SP_HIP_NO_LANE_ATTN", "1")
 
 
 @pytest.mark.parametrize("path", ["default", "general"])
 @pytest.mark.parametrize("n_q,H,n_ctx,hd,mob", ATTN_CASES)
 def test_fused_attention_matches_oracle(n_q, H, n_ctx, hd, mob, path, monkeypatch):
-    """The default launch runs the matrix-core kernel at hd 128 (K 5/5/4/3, V 3-bit),
-    the one-position-per-lane kernel at hd 64 and the general kernel at hd 256;
-    path "general" forces the general kernel everywhere. All meet 1e-3."""
+    """The default launch runs the matrix-core kernel (K 5/5/4/3, V 3-bit at hd 64, 128 and
+    256); path "general" forces the general kernel. All meet 1e-3."""
     if path == "general":
         general_kernel_only(monkeypatch)
-    elif hd == 256:
-        pytest.skip("the default launch at head_dim 256 is the general kernel (path general)")
     say(f"attn path={path} n_q={n_q} H={H} n_ctx={n_ctx} hd={hd} mob={mob}")
     k16, v16 = W.cfg2_kv(n_heads=H, n_pos=n_ctx, hd=hd, seed=n_ctx)
     q = W.cfg2_q(n_q=n_q, hd=hd, pos=n_ctx, seed=n_ctx + 1)
@@ -103,23 +99,22 @@ def test_fused_attention_matches_oracle(n_q, H, n_ctx, hd, mob, path, monkeypatc
 
 
 @pytest.mark.parametrize("path", ["default", "general"])
-@pytest.mark.parametrize("n_q,H,n_ctx,k_bits,v_bits,runs", [
-    (32, 32, 300, (5, 4, 4), (5,), 0),      # configs[2] (Phi-3-mini, MHA) at the bridge's hd-96 bands
-    (32, 32, 4096, (5, 4, 4), (5,), 0),     # configs[2]'s per-sequence shape: 64 tiles per head
-    (16, 4, 3000, (5, 4, 4), (5,), 3),      # GQA 4, runs of 15-16 tiles, a ragged last tile
-    (24, 8, 777, (5, 4, 4), (5,), 0),       # GQA 3
-    (16, 4, 1037, (5, 5, 4, 3), (3,), 0),   # the shipping bands at hd 96, GQA 4 (general kernel only)
+@pytest.mark.parametrize("n_q,H,n_ctx,k_bits,v_bits", [
+    (32, 32, 300, (5, 4, 4), (5,)),      # configs[2] (Phi-3-mini, MHA) at the bridge's hd-96 bands
+    (32, 32, 4096, (5, 4, 4), (5,)),     # configs[2]'s per-sequence shape: 64 tiles per head
+    (32, 32, 8300, (5, 4, 4), (5,)),     # 4160 tiles: two per wave on 256 CUs, a ragged last tile
+    (16, 4, 3000, (5, 4, 4), (5,)),      # GQA 4, a ragged last tile
+    (24, 8, 777, (5, 4, 4), (5,)),       # GQA 3
+    (16, 4, 1037, (5, 5, 4, 3), (3,)),   # the shipping bands at hd 96, GQA 4 (general kernel only)
 ])
-def test_hd96_attention_matches_oracle(n_q, H, n_ctx, k_bits, v_bits, runs, path, monkeypatch):
+def test_hd96_attention_matches_oracle(n_q, H, n_ctx, k_bits, v_bits, path, monkeypatch):
     """head_dim 96 (Vilenkin 2^5 * 3): the bridge's bands (K 5/4/4 + Mobius, V 5) run
-    the one-position-per-lane kernel by default, other bands the general kernel;
-    scores and output within 1e-3 of the oracle, several splits or runs and a ragged
-    last tile."""
+    the matrix-core kernel by default, other bands the general kernel; scores and output
+    within 1e-3 of the oracle, several blocks or splits, several tiles per wave and a
+    ragged last tile."""
     hd = 96
     if path == "general":
         general_kernel_only(monkeypatch)
-    if runs:
-        monkeypatch.setenv("SP_HIP_ATTN_LANE_RUNS", str(runs))
     say(f"attn hd96 path={path} n_q={n_q} H={H} n_ctx={n_ctx} k={k_bits} v={v_bits}")
     k16, v16 = W.cfg3_kv(n_heads=H, n_pos=n_ctx, hd=hd, seed=n_ctx)
     q = W.cfg2_q(n_q=n_q, hd=hd, pos=n_ctx, seed=n_ctx + 1)
@@ -196,11 +191,13 @@ def test_band_limited_attention_matches_oracle(n_q, H, n_ctx, path, monkeypatch)
 
 
 @pytest.mark.parametrize("hd,k_bits,v_bits,n_q,H,n_ctx", [
-    (96, (5, 4, 4), (5,), 8, 2, 700),        # configs[2]'s bands: the lane kernel's three K bands
+    (96, (5, 4, 4), (5,), 8, 2, 700),        # configs[2]'s bands: three K bands
     (64, (5, 5, 4, 3), (3,), 12, 4, 333),    # hd 64 shipping bands, GQA 3
+    (64, (5, 4, 4), (5,), 10, 2, 450),       # hd 64 at the bridge's bands, GQA 5
+    (256, (5, 5, 4, 3), (3,), 4, 2, 390),
 ])
-def test_lane_band_limited_attention_matches_oracle(hd, k_bits, v_bits, n_q, H, n_ctx):
-    """The one-position-per-lane kernel's band limits (sp_hip_attn_decode_bands): K bands
+def test_band_limited_attention_of_other_layouts_matches_oracle(hd, k_bits, v_bits, n_q, H, n_ctx):
+    """The matrix-core kernel's band limits (sp_hip_attn_decode_bands) at every head_dim: K bands
     past the limit, and V when the limit is 0, read as 0, against the oracle over the
     partial reconstructions (1e-3); the full band count and -1 equal the full call."""
     k16, v16 = W.cfg3_kv(n_heads=H, n_pos=n_ctx, hd=hd, seed=n_ctx + 5)
@@ -222,7 +219,7 @@ def test_lane_band_limited_attention_matches_oracle(hd, k_bits, v_bits, n_q, H, 
     S.check(L.sp_hip_attn_decode(cc.ref, 0, n_ctx, p(qt), n_q, C.c_float(scale), p(sc_full), p(out_full), stream()))
     nb = len(k_bits)
     for mb in list(range(nb)) + [nb, -1]:
-        say(f"lane attn bands hd={hd} n_q={n_q} H={H} n_ctx={n_ctx} max_bands={mb}")
+        say(f"attn bands hd={hd} n_q={n_q} H={H} n_ctx={n_ctx} max_bands={mb}")
         sc, out = empty_f32(n_q * n_ctx), empty_f32(n_q * hd)
         S.check(L.sp_hip_attn_decode_bands(cc.ref, 0, n_ctx, p(qt), n_q, C.c_float(scale), p(sc), p(out), mb,
                                            stream()))
@@ -241,11 +238,12 @@ def test_lane_band_limited_attention_matches_oracle(hd, k_bits, v_bits, n_q, H, 
 # CU): 8 KV heads at 32768 positions are 4096 tiles on 256 blocks, one tile per wave,
 # and a layer is one launch whose last block per KV head merges the blocks'
 # partials. 16600 (260 tiles per head, the last one partial) ends each head with a
-# partial tile. 40000 (625 tiles per head, 5000 in all) is more than one round, so
-# each wave walks two tiles with an online softmax across them (the multi-tile path).
+# partial tile. At 40000 (625 tiles per head, 5000 in all) the scores-only call walks
+# two tiles a wave in blocks of 16; at 50000 (6256 tiles, past 1.5 rounds) the calls
+# with an output walk four in blocks of four waves, with an online softmax across them.
 # (4, 1, 40000) and (8, 1, 40000): one KV head, so its blocks all count on one
 # counter and the last of them merges every block's partials.
-LONG_CASES = [(32, 8, 32768), (32, 8, 16600), (32, 8, 40000), (4, 1, 40000), (8, 1, 40000)]
+LONG_CASES = [(32, 8, 32768), (32, 8, 16600), (32, 8, 40000), (32, 8, 50000), (4, 1, 40000), (8, 1, 40000)]
 
 
 @functools.lru_cache(maxsize=1)

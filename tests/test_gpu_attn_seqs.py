@@ -55,13 +55,13 @@ def _check(fn, cache_ref, layer, starts, lens, q, n_q, hd, scale, ref_fn):
 
 SHIP_CASES = [
     # hd, K bits, V bits, H, n_q, starts, lens, max_seq
-    # the lane kernel, all five sequences in one launch (58- and 62-byte records at even
-    # starts of an even max_seq: dword-aligned bases)
+    # all five sequences in one launch of the matrix-core kernel, as in every case here (58-
+    # and 62-byte records at even starts of an even max_seq: dword-aligned bases)
     (96, (5, 4, 4), (5,), 4, 8, [0, 4096, 5200, 5200, 9000], [4096, 1000, 1, 2500, 64], 9068),
-    # an odd start (a base off dword alignment): one launch sequence per sequence
+    # an odd start (a base off dword alignment)
     (96, (5, 4, 4), (5,), 4, 8, [0, 3001, 700], [3001, 999, 2000], 4004),
-    (128, (5, 5, 4, 3), (3,), 2, 8, [0, 3000, 100], [3000, 1500, 700], 4503),  # matrix-core kernel per sequence
-    (64, (5, 5, 4, 3), (3,), 2, 4, [0, 600], [600, 333], 936),                  # the lane kernel at hd 64
+    (128, (5, 5, 4, 3), (3,), 2, 8, [0, 3000, 100], [3000, 1500, 700], 4503),
+    (64, (5, 5, 4, 3), (3,), 2, 4, [0, 600], [600, 333], 936),
 ]
 
 

@@ -98,3 +98,27 @@ def test_long_single_sequence_head_dim_64():
     rel_close(host(sc).reshape(n_q, n), s_ref)
     rel_close(host(out).reshape(n_q, hd), o_ref)
     cc.free()
+
+
+@pytest.mark.parametrize("G,n", [(1, 37001), (8, 37001), (4, 80000)])
+def test_scores_alone_of_long_sequences(G, n):
+    """One sequence past 9/8 of a round at head_dim 128: the scores alone go in blocks of 16 waves of
+    several tiles (two of 4632 tiles, three of 10000), with an output in other shapes; the
+    same scores bit for bit."""
+    hd, H = 128, 8
+    n_q = H * G
+    say(f"wave attn scores alone G={G} n={n}")
+    cc = S.ShipCache(S.config(hd, 1, H), n, stream=torch.cuda.current_stream().cuda_stream)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(n + G)
+    k, v = (torch.randn((n, H * hd), generator=g, device="cuda").half() for _ in range(2))
+    S.check(S.lib().sp_hip_write_layer(cc.ref, 0, 0, n, p(k), p(v), H * hd, S.DTYPE_F16))
+    q = torch.randn((n_q, hd), generator=g, device="cuda")
+    for mb in (-1, 2):
+        both, alone, out = empty_f32(n_q * n), empty_f32(n_q * n), empty_f32(n_q * hd)
+        args = (cc.ref, 0, n, p(q), n_q, C.c_float(1.0 / math.sqrt(hd)))
+        S.check(S.lib().sp_hip_attn_decode_bands(*args, p(both), p(out), mb, stream()))
+        S.check(S.lib().sp_hip_attn_decode_bands(*args, p(alone), None, mb, stream()))
+        assert torch.equal(both.view(torch.int32), alone.view(torch.int32))
+        assert bool(torch.isfinite(out).all()) and bool((out != 0).any())
+    cc.free()

@@ -73,22 +73,33 @@ def test_layer_calls_match_oracle(n, start, f32):
 
 
 def test_large_calls_match_small_ones():
-    """8 heads x 8200 positions, K and V: whole calls (2064 tiles: the one-wave kernels, four
-    rounds of a tile per SIMD, each block walking several) against calls of 1000 positions (the
-    block-per-tile kernels)."""
-    H, n, step = 8, 8200, 1000
+    """8 heads, K and V, eight tiles per CU (8185 positions on 256 CUs, a ragged last tile): whole
+    calls (the one-wave kernels, two whole rounds of a tile per SIMD where the block-per-tile
+    ones take eight of a tile per CU: the rule's line is 3.2 to one) against calls of 1000
+    positions (the block-per-tile kernels), and the whole call's first and last records of a
+    head against the oracle."""
+    H, step = 8, 1000
+    n = 32 * torch.cuda.get_device_properties(0).multi_processor_count - 7
     say(f"hier split vs lane n={n}")
     g = torch.Generator(device="cuda")
     g.manual_seed(3)
     x = [torch.randn((n, H * HD), generator=g, device="cuda").half() for _ in range(2)]
-    whole, parts = _cache(H, n)[0], _cache(H, n)[0]
+    (whole, Wm), (parts, _) = _cache(H, n), _cache(H, n)
     L = S.lib()
     S.check(L.sp_hip_hier_write_layer(whole.ref, 0, 0, n, p(x[0]), p(x[1]), H * HD, S.DTYPE_F16))
     for a in range(0, n, step):
         m = min(step, n - a)
         S.check(L.sp_hip_hier_write_layer(parts.ref, 0, a, m, p(x[0][a:]), p(x[1][a:]), H * HD, S.DTYPE_F16))
-    for a, b in zip(_records(whole, H, n), _records(parts, H, n)):
+    recs = _records(whole, H, n)
+    for a, b in zip(recs, _records(parts, H, n)):
         np.testing.assert_array_equal(a, b)
+    sk, tg = O.hier_geometry(PAD)
+    ends = np.r_[0:70, n - 70:n]
+    for side in range(2):
+        for h in (0, H - 1):
+            rows = x[side].view(n, H, HD)[:, h].cpu().numpy()[ends]
+            ref = O.hier_compress_f16(np.ascontiguousarray(rows).view(np.uint16), HD, PAD, sk, tg, O.band_config(len(sk), [5, 5]), Wm[h], 2)
+            np.testing.assert_array_equal(recs[side][h, ends], ref)
     y = [torch.zeros_like(x[0]) for _ in range(4)]
     S.check(L.sp_hip_hier_read_layer(whole.ref, 0, 0, n, p(y[0]), p(y[1]), H * HD, S.DTYPE_F16))
     for a in range(0, n, step):
