@@ -204,13 +204,9 @@ __device__ __forceinline__ void split_hl(float v, uint32_t &hi, uint32_t &lo) {
 // every zero), what it scales still has its fp32 precision down to about 2^-126, and a wave
 // that has seen no weight yet keeps the largest p there is, so the first one sets its own.
 __device__ __forceinline__ float pow2_norm(float amax, float &inv) {
-    if (!(amax < INFINITY)) {
-        inv = 1.0f;
-        return 1.0f;
-    }
     int e;
-    (void)frexpf(amax, &e);  // amax = f * 2^e, f in [0.5, 1)
-    e = amax > 0.0f ? max(e, -112) : -112;
+    (void)frexpf(fmaxf(amax, 0x1p-113f), &e);  // the larger one = f * 2^e, f in [0.5, 1)
+    e = amax < INFINITY ? e : 12;
     inv = ldexpf(1.0f, e - 12);
     return ldexpf(1.0f, 12 - e);
 }
@@ -775,16 +771,17 @@ k_attn_wave(const SpAttnArgs A, const int *__restrict__ order, float *__restrict
             for (int i = 0; i < 4; i++) v[st][i] = 4 * qd + i < n_chunk ? sc[st][i] : -INFINITY;  // past the tile's end: no weight
             grown[st] = false;
             if (MULTI) {
-                float wm = 0.0f, pm = 0.0f;
+                float wm = 0.0f;
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
                     pr[st][i] = __expf(v[st][i] - m_run[st]);
                     wx[st][i] = pr[st][i] * sv[i] * f_run[st];
                     wm = fmaxf(wm, wx[st][i]);
-                    pm = fmaxf(pm, pr[st][i]);
                 }
-                // both bounds in one: 2^60 * 2^-45 is 2^15 (and an infinite p passes it)
-                grown[st] = 4 * st + hj < G && !(fmaf(pm, 0x1p-45f, wm) <= 32768.0f);
+                // both bounds in one, p's on the lane's sum: 2^60 * 2^-45 is 2^15 (and an infinite p
+                // passes it)
+                const float ps = (pr[st][0] + pr[st][1]) + (pr[st][2] + pr[st][3]);
+                grown[st] = 4 * st + hj < G && !(fmaf(ps, 0x1p-45f, wm) <= 32768.0f);
                 any_grown = any_grown || grown[st];
             }
         }
