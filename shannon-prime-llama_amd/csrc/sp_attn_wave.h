@@ -198,17 +198,21 @@ __device__ __forceinline__ void split_hl(float v, uint32_t &hi, uint32_t &lo) {
     lo = (uint32_t)__builtin_bit_cast(unsigned short, l);
 }
 
-// Power of two p with amax * p in [2^11, 2^12) (1 when amax is not finite), and its
-// reciprocal (exact). An amax below 2^-113, zero too, takes the p of 2^-113: p and 1/p, also
-// with the weights' 2^-6 on them, stay normal numbers (an infinite p would make a NaN of
-// every zero), what it scales still has its fp32 precision down to about 2^-126, and a wave
-// that has seen no weight yet keeps the largest p there is, so the first one sets its own.
+// Power of two p with amax * p in [2^11, 2^12), and its reciprocal (both exact). An amax below
+// 2^-113, zero too, takes the p of 2^-113: p and 1/p, also with the weights' 2^-6 on them, stay
+// normal numbers (an infinite p would make a NaN of every zero), what it scales still has its
+// fp32 precision down to about 2^-126, and a wave that has seen no weight yet keeps the largest
+// p there is, so the first one sets its own. An infinite amax takes the largest number's p.
+// (The clamp is one v_med3, but for two head sets at head_dim 256: there it had the register
+// allocator spill eight more, 16 sequences of up to 2000 positions 42.4 us against 40.8.
+// With fminf and fmaxf at head_dim 96 it spilled eight: 16 x 4096 positions 54.7 -> 59.)
+template <class LY, int NH>
 __device__ __forceinline__ float pow2_norm(float amax, float &inv) {
-    int e;
-    (void)frexpf(fmaxf(amax, 0x1p-113f), &e);  // the larger one = f * 2^e, f in [0.5, 1)
-    e = amax < INFINITY ? e : 12;
-    inv = ldexpf(1.0f, e - 12);
-    return ldexpf(1.0f, 12 - e);
+    constexpr float lo = 0x1p-113f, hi = 0x1.fffffep127f;
+    const float a = LY::HD == 256 && NH == 2 ? fminf(fmaxf(amax, lo), hi) : __builtin_amdgcn_fmed3f(amax, lo, hi);
+    const uint32_t E = __float_as_uint(a) & 0x7f800000u;  // a = f * 2^e, f in [0.5, 1): e + 126 in place
+    inv = __uint_as_float(E - (11u << 23));               // 2^(e - 12)
+    return __uint_as_float((265u << 23) - E);             // 2^(12 - e)
 }
 
 // fp16 scale bits -> float; a non-finite scale dequantizes to 0.
@@ -564,7 +568,7 @@ k_attn_wave(const SpAttnArgs A, const int *__restrict__ order, float *__restrict
         amax = wave_max_step<16>(amax);
         amax = wave_max_step<32>(amax);
         float finv;
-        const float f = pow2_norm(amax, finv);
+        const float f = pow2_norm<LY, NH>(amax, finv);
         // reorder through the wave's (not yet used) record area; clear the row's pad slots
         float *qx = reinterpret_cast<float *>(wl);
 #pragma unroll
@@ -771,17 +775,16 @@ k_attn_wave(const SpAttnArgs A, const int *__restrict__ order, float *__restrict
             for (int i = 0; i < 4; i++) v[st][i] = 4 * qd + i < n_chunk ? sc[st][i] : -INFINITY;  // past the tile's end: no weight
             grown[st] = false;
             if (MULTI) {
-                float wm = 0.0f;
+                float wm = 0.0f, pm = 0.0f;
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
                     pr[st][i] = __expf(v[st][i] - m_run[st]);
                     wx[st][i] = pr[st][i] * sv[i] * f_run[st];
                     wm = fmaxf(wm, wx[st][i]);
+                    pm = fmaxf(pm, pr[st][i]);
                 }
-                // both bounds in one, p's on the lane's sum: 2^60 * 2^-45 is 2^15 (and an infinite p
-                // passes it)
-                const float ps = (pr[st][0] + pr[st][1]) + (pr[st][2] + pr[st][3]);
-                grown[st] = 4 * st + hj < G && !(fmaf(ps, 0x1p-45f, wm) <= 32768.0f);
+                // both bounds in one: 2^60 * 2^-45 is 2^15 (and an infinite p passes it)
+                grown[st] = 4 * st + hj < G && !(fmaf(pm, 0x1p-45f, wm) <= 32768.0f);
                 any_grown = any_grown || grown[st];
             }
         }
@@ -797,7 +800,7 @@ k_attn_wave(const SpAttnArgs A, const int *__restrict__ order, float *__restrict
                     wm = fmaxf(wm, p[i] * sv[i]);
                 }
                 float fi;
-                const float f = pow2_norm(head_max(wm), fi) * 0.015625f;
+                const float f = pow2_norm<LY, NH>(head_max(wm), fi) * 0.015625f;
                 fi *= 64.0f;
                 const float alpha = !MULTI || it == 0 ? 0.0f : __expf(m_run[st] - m);
                 // what the head's value sums are multiplied by
