@@ -19,15 +19,18 @@ from test_gpu_attn_seqs import _arr  # noqa: E402
 from test_gpu_attn_wave import BRIDGE, LAYOUTS, SHIP  # noqa: E402
 
 
-def _run(hd, bands, H, n_q, score, v_amp, n_seq=1, q_scale=1.0):
+def _run(hd, bands, H, n_q, score, v_amp, n_seq=1, q_scale=1.0, broken=()):
     """n_seq equal sequences over the same cells: position t scores score[t] for every query head
     and its V row is v_amp[t] * N(0, 1). The cache has cells for all of them (its workspace is
-    sized by them), so they go out in one launch."""
+    sized by them), so they go out in one launch. broken: (position, K value, V value) put into
+    a row's element."""
     n = len(score)
     rng = np.random.default_rng(hd + n)
     u = rng.standard_normal((H, 1, hd)) / 10
     k16 = (u * np.asarray(score)[None, :, None]).astype(np.float16)
     v16 = (rng.standard_normal((H, n, hd)) * np.asarray(v_amp)[None, :, None]).astype(np.float16)
+    for t, kv, vv in broken:
+        k16[:, t, 3], v16[:, t, hd - 2] = kv, vv
     kbc, vbc, order = O.band_config(hd, list(bands[0])), O.band_config(hd, list(bands[1])), O.mobius_order(hd)
     kr = O.ship_compress_f16(k16.reshape(-1, hd).view(np.uint16), kbc, order).reshape(H, n, -1)
     vr = O.ship_compress_f16(v16.reshape(-1, hd).view(np.uint16), vbc).reshape(H, n, -1)
@@ -99,3 +102,14 @@ def test_later_best_position_without_values(hd, bands, H, G, n_seq, n, above):
     score[7 * 64 + 21], v_amp[7 * 64 + 21] = -0.5, 0.0
     score[16 * 64 + 5:16 * 64 + 9] = -3.5
     _run(hd, bands, H, H * G, score, v_amp, n_seq)
+
+
+@pytest.mark.parametrize("hd,bands,H,G,n_seq,n", SEVERAL)
+def test_rows_that_are_not_finite(hd, bands, H, G, n_seq, n):
+    """K and V rows with an infinity or a NaN, in the first, a middle and the last tile: their bands'
+    scales are not finite, which reads as 0, at positions that would have scored among the best."""
+    say(f"wave attn rows not finite hd={hd} bands={bands} H={H} G={G} n={n}")
+    score = np.linspace(-3.0, -0.5, n)
+    _run(hd, bands, H, H * G, score, np.ones(n), n_seq,
+         broken=[(5, np.inf, 1.0), (9, 1.0, -np.inf), (n // 2, -np.inf, np.inf), (n // 2 + 1, 1.0, np.nan), (n - 2, 1.0, np.inf),
+                 (n - 1, np.inf, np.nan)])
