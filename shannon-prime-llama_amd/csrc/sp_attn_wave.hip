@@ -40,7 +40,7 @@ static int wave_device_cus() {
 // one sequence of 250 to 40000 positions they are within 10% of the best of the three sizes but
 // for 5000 tiles at one tile per wave (8 waves would be 15-25% faster than 16). Batches of
 // short sequences with 5 to 8 heads per KV head would be up to twice as fast in blocks of 16
-// (12 of up to 600 positions: 25.9 us, 12.2): the last block's merge is a round per block's threads.
+// (12 of up to 600 positions: 25.9 us, 12.2): a last block of 4 merges eight heads in four rounds.
 struct WaveShape {
     int nw, tpw;
 };
